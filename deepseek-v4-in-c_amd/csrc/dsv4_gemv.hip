@@ -125,65 +125,169 @@ static hipError_t launch_fmt(const GemvArgs &a, hipStream_t st)
 
 /* ------------------------------------------------------------- BF16 --- */
 
-/* One wave per ROWS rows: the rows go to LDS once, then for every token its
- * x goes to LDS and the rows' dot products run from there. ROWS x (1 KiB KCH
- * + 64) bytes of rows (64: a bank offset between rows), then up to 2 KiB
- * KCH of x. */
-constexpr int BF16_PAD = 64;
-template <int KCH, int ROWS>
-__host__ __device__ constexpr size_t bf16_gemv_lds() { return (size_t)ROWS * (KCH * 1024 + BF16_PAD) + 2048 * KCH; }
-
-template <int KCH, int ROWS>
-__global__ __launch_bounds__(64) void k_gemv_bf16(GemvBf16Args a)
+/* One to four tokens, many rows: a wave's 8 RG rows straight from memory to
+ * registers, D steps of 64 columns in flight. Waves are independent. Bound by
+ * HBM: the [129280 x 4096] head, one token, 284 -> 178 us (3.7 -> 6.0 TB/s)
+ * against a wave that staged its rows and x in LDS and ran each chain as
+ * dependent fp64 FMAs. RG = 2 halves the x loads per weight (RG = 1: 222 us;
+ * RG = 4, with half the waves, 226), D = 2 / 4 / 8: 182 / 179 / 177. */
+template <int RG, int D>
+__global__ __launch_bounds__(256) void k_gemv_bf16(GemvBf16Args a)
 {
-    extern __shared__ __align__(16) uint8_t lds[];
-    const int lane = threadIdx.x;
-    const int r0 = blockIdx.x * ROWS;
-    constexpr int STRIDE = KCH * 1024 + BF16_PAD;
-    uint8_t *xl = lds + ROWS * STRIDE;
-    bf16_rows_to_lds<KCH>(lds, STRIDE, a.W, r0, ROWS, a.rows - r0, 2 * a.cols, lane);
-    const int r = lane >> 4;
-    const uint16_t *wl = (const uint16_t *)(lds + (r < ROWS ? r : 0) * STRIDE);
-    for (int t = 0; t < a.nt; t++) {
-        /* a single wave: its reads of the previous token's x are done */
-        bf16_x_to_lds(xl, a.x + (size_t)t * a.x_ld, a.cols, lane);
-        __builtin_amdgcn_s_waitcnt(0x0F70);          /* vmcnt(0): rows and x landed */
-        asm volatile("" ::: "memory");
-        const double acc = bf16_row_dot(wl, (const float *)xl, a.cols, lane);
-        if (r < ROWS && (lane & 15) == 0 && r0 + r < a.rows) a.y[(size_t)t * a.y_ld + r0 + r] = (float)acc;
+    typedef Bf16Tile<RG> Tile;
+    const int lane = threadIdx.x & 63;
+    const int r0 = wave_id() * (Tile::ROWS * RG);
+    if (r0 >= a.rows) return;
+    Tile tile;
+    tile.init(a.W, r0, a.rows, a.x, a.x_ld, a.nt, a.cols, lane);
+    tile.template chains<D>(a.cols, lane);
+    const int tok = lane & 3;
+    const float *xrow = a.x + (size_t)min(tok, a.nt - 1) * a.x_ld;
+#pragma unroll
+    for (int r = 0; r < RG; r++) {
+        const int row = r0 + Tile::ROWS * r + Tile::out_row(lane);
+        const double v = tile.finish(r, a.W + (size_t)min(row, a.rows - 1) * a.cols, xrow, a.cols);
+        if (!(lane & 4) && row < a.rows && tok < a.nt) a.y[(size_t)tok * a.y_ld + row] = (float)v;
     }
 }
 
-template <int KCH, int ROWS>
-static hipError_t launch_bf16_k(const GemvBf16Args &a, hipStream_t st)
+/* Few tokens, few rows: four rows and four tokens per workgroup. Bound by
+ * latency: the [256 x 4096] gate, 8 tokens, 42.3 -> 6.8 us. */
+__global__ __launch_bounds__(256) void k_gemv4_bf16(GemvBf16Args a)
 {
-    constexpr size_t lds = bf16_gemv_lds<KCH, ROWS>();
-    if constexpr (lds > 64 * 1024) {
-        /* set once (not inside a stream capture of a later call) */
-        static bool set = false;
-        if (!set) {
-            const hipError_t e = hipFuncSetAttribute((const void *)k_gemv_bf16<KCH, ROWS>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-            set = true;
+    extern __shared__ __align__(16) uint8_t b4_lds[];
+    const int r0 = 4 * blockIdx.x, t0 = 4 * blockIdx.y;
+    const double v = bf16_dot4(b4_lds, a.W, r0, a.rows, a.x + (size_t)t0 * a.x_ld, a.x_ld, min(4, a.nt - t0), a.cols);
+    const int tid = threadIdx.x, row = r0 + (tid >> 4), tok = t0 + (tid & 3);
+    if (tid < 64 && !(tid & 12) && row < a.rows && tok < a.nt) a.y[(size_t)tok * a.y_ld + row] = (float)v;
+}
+
+/* Many tokens: 16 rows x 16 tokens per workgroup on v_mfma_f64_16x16x4 (64
+ * cycles), wave w of four running chains 4 w .. 4 w + 3. 256 columns of the
+ * rows and the tokens at a time go through LDS (two stages, direct loads);
+ * the chains meet in LDS at the end. Bound by the fp64 matrix rate with many
+ * tokens (the gate [256 x 4096], 701 tokens: 3,890 -> 34 us, 19 us of it MFMA
+ * issue at 2.4 GHz), by the 16 stages' latency with few (15 us). */
+constexpr int BFG_COLS = 256;
+constexpr int BFG_A_LD = 1024 + 16;                /* two rows of 512 bytes, then a bank offset */
+constexpr int BFG_B_LD = 1024 + 16;                /* one token of 1024 bytes                    */
+constexpr int BFG_STAGE = 8 * BFG_A_LD + 16 * BFG_B_LD;
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(256) void k_gemm_bf16(GemvBf16Args a)
+{
+    __shared__ __align__(16) uint8_t lds[2 * BFG_STAGE];
+    static_assert(2 * BFG_STAGE >= 4 * 16 * 64 * 8, "the chains' exchange");
+    const int lane = threadIdx.x & 63, wv = wave_in_group();
+    const int lr = lane & 15, lk = lane >> 4;
+    const int nrb = (a.rows + 15) / 16;
+    const int t0 = blockIdx.x / nrb * 16, r0 = blockIdx.x % nrb * 16;
+    const int cols16 = a.cols / 16 * 16;
+    const int nstage = (cols16 + BFG_COLS - 1) / BFG_COLS;
+    const int nr = min(16, a.rows - r0), nt = min(16, a.nt - t0);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(a.W + (size_t)r0 * a.cols), (short)0, nr * a.cols * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(a.x + (size_t)t0 * a.x_ld), (short)0, ((nt - 1) * a.x_ld + a.cols) * 4, 0x00020000);
+    /* columns past cols16 answer with zeros (an offset past the resource);
+     * rows and tokens past the end repeat the last */
+    const int none = 0x7FFFFFF0;
+    auto load = [&](int st) {
+        uint8_t *base = lds + (st & 1) * BFG_STAGE;
+        const int c0 = st * BFG_COLS;
+#pragma unroll
+        for (int i = 0; i < 2; i++) {              /* row pairs wv and wv + 4 */
+            const int p = wv + 4 * i, row = min(2 * p + (lane >> 5), nr - 1), c = c0 + 8 * (lane & 31);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (bf_lds_t *)(base + p * BFG_A_LD), 16,
+                                                     c < cols16 ? (row * a.cols + c) * 2 : none, 0, 0, 0);
         }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {              /* tokens wv + 4 i */
+            const int p = wv + 4 * i, tok = min(p, nt - 1), c = c0 + 4 * lane;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (bf_lds_t *)(base + 8 * BFG_A_LD + p * BFG_B_LD), 16,
+                                                     c < cols16 ? (tok * a.x_ld + c) * 4 : none, 0, 0, 0);
+        }
+    };
+    f64x4 acc[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) acc[q] = f64x4{0.0, 0.0, 0.0, 0.0};
+    load(0);
+    __syncthreads();
+    for (int st = 0; st < nstage; st++) {
+        if (st + 1 < nstage) load(st + 1);
+        const uint8_t *base = lds + (st & 1) * BFG_STAGE;
+        const uint8_t *pa = base + (lr >> 1) * BFG_A_LD + (lr & 1) * 512 + 2 * (16 * lk + 4 * wv);
+        const uint8_t *pb = base + 8 * BFG_A_LD + lr * BFG_B_LD + 4 * (16 * lk + 4 * wv);
+#pragma unroll
+        for (int s = 0; s < BFG_COLS / 64; s++) {
+            const u32x2 w = *(const u32x2 *)(pa + 128 * s);
+            const f32x4 x = *(const f32x4 *)(pb + 256 * s);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf16_elem(w, q), (double)x[q], acc[q], 0, 0, 0);
+        }
+        __syncthreads();                           /* the next stage has landed, this one is free */
     }
-    hipLaunchKernelGGL((k_gemv_bf16<KCH, ROWS>), dim3((unsigned)((a.rows + ROWS - 1) / ROWS)), dim3(64), lds,
-                       st, a);
-    return hipGetLastError();
+    /* element e of chain q, lane l: row 4 e + l / 16, token l % 16. Wave w
+     * combines the elements e = w: chain j is wave j / 4's q = j % 4. */
+    double *xc = (double *)lds;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) xc[((wv * 4 + q) * 4 + e) * 64 + lane] = acc[q][e];
+    __syncthreads();
+    double bb[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        double c[4];
+#pragma unroll
+        for (int w = 0; w < 4; w++) c[w] = xc[((w * 4 + q) * 4 + wv) * 64 + lane];
+        bb[q] = (c[0] + c[1]) + (c[2] + c[3]);
+    }
+    double v = (bb[0] + bb[1]) + (bb[2] + bb[3]);
+    const int row = 4 * wv + lk;
+    if (row >= nr || lr >= nt) return;
+    const uint16_t *wr = a.W + (size_t)(r0 + row) * a.cols;
+    const float *xr = a.x + (size_t)(t0 + lr) * a.x_ld;
+    for (int e = cols16; e < a.cols; e++) v = fma(bf16_of(wr[e]), (double)xr[e], v);
+    a.y[(size_t)(t0 + lr) * a.y_ld + r0 + row] = (float)v;
 }
 
+/* Which form, all three with the same bits. us at 4096 columns for (small /
+ * rows / GEMM), measured: 1 token: 1024 rows 6.4 / 20 / 15, 8192 rows 18.8 /
+ * 22 / 25, 16384 rows 37 / 25 / 45; 4 tokens: 256 rows 6.7 / - / 15, 4096
+ * rows 20 / 31 / 16, 8192 rows 37 / 31 / 26, 32768 rows 147 / 61 / 88; 32
+ * tokens: 256 rows 10.1 / - / 15, 1024 rows 36 / - / 15. So: the rows form
+ * for a few tokens of a large matrix, the small form while its workgroups
+ * run in at most three rounds of what LDS lets the device hold at once, else
+ * the GEMM. */
 hipError_t gemv_bf16_launch(const GemvBf16Args &a, hipStream_t st)
 {
     if (a.rows <= 0 || a.cols <= 0 || a.cols % 8 || a.nt <= 0) return hipErrorInvalidValue;
-    switch ((2 * a.cols + 1023) / 1024) {
-    case 1: return launch_bf16_k<1, 4>(a, st);
-    case 2: return launch_bf16_k<2, 4>(a, st);
-    case 3: case 4: return launch_bf16_k<4, 4>(a, st);
-    case 5: case 6: case 7: case 8: return launch_bf16_k<8, 4>(a, st);
-    case 9: case 10: case 11: case 12: case 13: case 14: case 15: case 16: return launch_bf16_k<16, 4>(a, st);
-    default: return hipErrorInvalidValue;
+    if (a.nt <= 4 && a.rows >= (a.nt == 1 ? 9216 : 12288)) {
+        constexpr int RG = 2;
+        const int waves = (a.rows + 8 * RG - 1) / (8 * RG);
+        hipLaunchKernelGGL((k_gemv_bf16<RG, 8>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, a);
+        return hipGetLastError();
     }
+    const int lds = b4_lds_bytes(a.nt < 4 ? a.nt : 4);
+    const long small = (((long)a.rows + 3) / 4) * (((long)a.nt + 3) / 4);
+    if (small <= 3L * 256 * (160 * 1024 / lds)) {
+        static bool attr_done = false;             /* not again inside a stream capture of a later call */
+        if (!attr_done) {
+            const hipError_t e = hipFuncSetAttribute((const void *)k_gemv4_bf16,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, b4_lds_bytes(4));
+            if (e != hipSuccess) return e;
+            attr_done = true;
+        }
+        hipLaunchKernelGGL(k_gemv4_bf16, dim3((unsigned)((a.rows + 3) / 4), (unsigned)((a.nt + 3) / 4)), dim3(256),
+                           lds, st, a);
+        return hipGetLastError();
+    }
+    const long grid = (((long)a.nt + 15) / 16) * (((long)a.rows + 15) / 16);
+    if (grid > 0x7FFFFFFF) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_gemm_bf16, dim3((unsigned)grid), dim3(256), 0, st, a);
+    return hipGetLastError();
 }
 
 hipError_t gemv_launch(int fmt, const GemvArgs &a, hipStream_t st)

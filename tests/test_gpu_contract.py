@@ -115,6 +115,26 @@ def test_bf16_gemv_special_values(lib, pkg, oracle, rows, cols, nt):
     m.drop()
 
 
+@pytest.mark.parametrize("rows,cols,nt", [
+    (9215, 72, 1), (9216, 1032, 1), (9223, 4096, 1),      # the rows form from 9216 rows, one token
+    (12287, 136, 3), (12301, 1096, 4), (12288, 24, 2),    # and from 12288 for two to four
+    (5, 4104, 4), (6, 8192, 5), (30, 8184, 8), (4, 16, 1),      # small form: one and two parts of columns
+    (2048, 264, 4), (2052, 264, 4), (1021, 264, 8),       # small form's and GEMM's sides of the three rounds
+    (17, 4104, 529), (3100, 264, 9), (3073, 520, 17), (3085, 8, 32)])
+def test_bf16_forms(lib, pkg, oracle, rows, cols, nt):
+    """Each form of the BF16 matvec at its edges: rows and tokens past the
+    last tile, one to three 16-column groups past the last 64, trailing 8
+    columns, no whole group; bit for bit bf16_n."""
+    rng = np.random.default_rng(rows * 11 + cols * 3 + nt)
+    W = bf16_bits(rng.standard_normal(rows * cols).astype(np.float32) * np.float32(0.02))
+    x = rng.standard_normal(nt * cols).astype(np.float32)
+    x[::7] *= np.float32(2.0 ** 40)        # products far apart, so that the order of the sums shows
+    x[::11] *= np.float32(2.0 ** -40)
+    m = ResidentBf16(lib, pkg, W, rows, cols)
+    check_bf16(lib.mmq_n(m.desc, x, nt), oracle.bf16_n(W, x, rows, cols, nt))
+    m.drop()
+
+
 # ------------------------------------------------------- wide FP8 rows ----
 
 @pytest.mark.parametrize("rows,nt", [(4096, 1), (1024, 1), (512, 3), (512, 40)])
