@@ -361,7 +361,8 @@ hipError_t synth_normal_launch(float *out, size_t n, uint64_t seed, float sigma,
 /* One token tile of the grouped GEMMs: its bucket (expert), first bucket
  * row and rows, so a workgroup finds its work in one load. */
 struct TileRec {
-    int grp, r0, ntok, pad;
+    int grp, r0, ntok;
+    int bucket;               /* rows of the tile's whole bucket          */
 };
 
 /* counting sort of the npairs = n * topk routing ids by expert; rows inside
@@ -455,7 +456,11 @@ struct GroupedArgs {
     float limit;
     unsigned *status;
 };
+/* tt: 1 or 4 (16- or 64-row tiles), 8 (128-row, FP4) or GROUPED_STREAM
+ * (16-row, FP4 experts of a table, geometry as grouped_stream_ok) */
+constexpr int GROUPED_STREAM = 5;
 int grouped_rows_per_tile(int tt);
+bool grouped_stream_ok(long nrows, int K, int N);
 hipError_t grouped_launch(int fmt, bool swiglu, int tt, const GroupedArgs &a, long max_tiles,
                           hipStream_t st);
 

@@ -350,7 +350,7 @@ __global__ __launch_bounds__(1024) void k_moe_route(RouteArgs a, int cpb)
         rec.grp = lo;
         rec.r0 = r0;
         rec.ntok = min(a.tile_rows, scan_r[lo] - r0);
-        rec.pad = 0;
+        rec.bucket = scan_r[lo] - go;
         a.tile_rec[t] = rec;
     }
     if (tid < E) {
@@ -1093,9 +1093,9 @@ __global__ __launch_bounds__(512) void k_grouped3(GroupedArgs a)
     }
     const int f0 = slab * FEAT;
     const int K = a.K, N = a.N;
-    /* buffer loads need 16-byte aligned weights and 4-byte aligned scales */
-    const bool aligned = ((uintptr_t)m1.w & 15) == 0 && ((uintptr_t)m1.s & 3) == 0 &&
-                         (!SWIGLU || (((uintptr_t)m3.w & 15) == 0 && ((uintptr_t)m3.s & 3) == 0));
+    /* buffer loads need dword-aligned weights and scales */
+    const bool aligned = (((uintptr_t)m1.w | (uintptr_t)m1.s) & 3) == 0 &&
+                         (!SWIGLU || (((uintptr_t)m3.w | (uintptr_t)m3.s) & 3) == 0);
     if (!qmat_matches<FMT_FP4_E8M0>(m1, N, K) || (SWIGLU && !qmat_matches<FMT_FP4_E8M0>(m3, N, K)) ||
         !aligned) {
         if (threadIdx.x == 0) atomicOr(a.status, ST_BAD_DESCRIPTOR);
@@ -1251,6 +1251,237 @@ __global__ __launch_bounds__(512) void k_grouped3(GroupedArgs a)
     if (range_bad) atomicOr(a.status, range_bad);
 }
 
+/* -------------------------------- FP4 weights streamed to registers --- */
+
+/* For buckets of up to a few dozen tokens, where an expert's weights are used
+ * so few times that streaming them is the bound (the batched decode, short
+ * prompts). Workgroup: four waves, a tile of 16 token rows. Each wave owns 16
+ * rows of each of two 64-row halves (gate/up: the w1 rows and the matching w3
+ * rows; down: rows f0 .. f0 + 63 and f0 + 64 .. f0 + 127) over all of K. A
+ * step is 256 reduction indices (128 bytes of a row), a group two steps: two
+ * groups of weights are in flight straight to registers, and the tile's token
+ * rows (fp16) of the same steps pass through four LDS slots, every wave
+ * loading its share in the same order as its weights, so that one counted
+ * wait covers both.
+ *
+ * A load instruction reads whole 128-byte lines of eight rows: lane
+ * 16 g + 2 r + h takes bytes 64 h + 16 g of row 2 r + j (j the instruction),
+ * and a lane-pair exchange forms the MFMA operands of rows 2 r + h. The
+ * reduction order, and so the bits, are k_grouped2's. The rows' E8M0 bytes
+ * go to LDS once, 8-byte pieces (a step's) XOR-swizzled by the row so that
+ * the 16 rows of a read start in distinct banks.
+ *
+ * Measured, 64 tokens x top-6 of 256 experts (Zipf), hidden 4096, inter 2048:
+ * gate/up 217 -> 172 us (6.1 TB/s), down 108 -> 92 us against k_grouped2,
+ * which passes the weights through LDS a step at a time. What decided: 256
+ * contiguous bytes of a row asked for together (one step at a time: 210 and
+ * 105), three workgroups a CU (113 registers, 48 KB of LDS; two: 352 against
+ * 322 us for the call), weights that nothing else reads loaded non-temporal,
+ * and few vector operations per weight (scale bytes shifted into place and
+ * checked once at the end). */
+namespace {
+
+constexpr int GW_G = 2;                            /* steps per group                     */
+constexpr int GW_XI = 2;                           /* token load instructions, wave, step */
+constexpr int GW_VM = GW_G * (4 + GW_XI);          /* loads per wave and group            */
+constexpr int GW_SLOT = 16 * KS * 2;               /* a step's 16 token rows              */
+constexpr int GW_KMAX = 8192;
+static_assert(GW_VM <= 15, "the wait below encodes vmcnt in four bits");
+constexpr int gw_lds(int K) { return 2 * GW_G * GW_SLOT + 128 * (K / 32); }
+
+constexpr int CPOL_NT = 2;                         /* non-temporal */
+template <int CPOL>
+__device__ __forceinline__ u32x4 bload16(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff)
+{
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, soff, CPOL));
+}
+
+/* whether one of four E8M0 bytes lies outside 104..140 */
+__device__ __forceinline__ bool scales_bad(uint32_t s)
+{
+    bool bad = false;
+#pragma unroll
+    for (int b = 0; b < 4; b++) bad |= ((s >> (8 * b)) & 0xFFu) - 104u > 36u;
+    return bad;
+}
+
+} // namespace
+
+template <bool SWIGLU>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_grouped_w(GroupedArgs a)
+{
+    constexpr int FEAT = SWIGLU ? 64 : 128;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = wave_in_group();
+    const int rr = lane & 15, gq = lane >> 4;
+    const int nslab = a.N / FEAT;
+    const int tile = blockIdx.x / nslab, slab = blockIdx.x - tile * nslab;
+    const int ntiles = ld_uniform(a.tile_pre, a.n_experts);
+    const TileRec tr = ld_uniform(a.tile_rec, tile);      /* read beside the count: one round trip */
+    if ((tile >= ntiles) | (tr.ntok <= 0)) return;        /* whole workgroup */
+    const int r0 = tr.r0, ntok = tr.ntok;
+    const DSV4ExpertW e = ld_uniform(a.table, tr.grp);
+    const DSV4QMat m1 = SWIGLU ? e.w1 : e.w2, m3 = e.w3;
+    const int f0 = slab * FEAT;
+    const int K = a.K, N = a.N;
+    if (!qmat_matches<FMT_FP4_E8M0>(m1, N, K) || (SWIGLU && !qmat_matches<FMT_FP4_E8M0>(m3, N, K))) {
+        if (threadIdx.x == 0) atomicOr(a.status, ST_BAD_DESCRIPTOR);
+        const float nan = __builtin_nanf("");
+        for (int i = threadIdx.x; i < ntok * FEAT; i += 256) {
+            const size_t o = (size_t)(r0 + i / FEAT) * N + f0 + i % FEAT;
+            if constexpr (SWIGLU) ((uint16_t *)a.out)[o] = (uint16_t)f16_bits(nan);
+            else ((float *)a.out)[o] = nan;
+        }
+        return;
+    }
+    /* groups rounded up to an even count: steps past the end multiply zeros */
+    const int nst = K / KS, ngr = (nst + 2 * GW_G - 1) / (2 * GW_G) * 2;
+    /* the two halves' rows: f0 .. f0 + 63 of m1 and of m3, or the next 64 of m1 */
+    const uint32_t rowb = (uint32_t)K / 2, srow = (uint32_t)K / 32;
+    const uint8_t *wb[2] = {(const uint8_t *)m1.w + (size_t)f0 * rowb,
+                            SWIGLU ? (const uint8_t *)m3.w + (size_t)f0 * rowb
+                                   : (const uint8_t *)m1.w + (size_t)(f0 + 64) * rowb};
+    const uint8_t *sb[2] = {(const uint8_t *)m1.s + (size_t)f0 * srow,
+                            SWIGLU ? (const uint8_t *)m3.s + (size_t)f0 * srow
+                                   : (const uint8_t *)m1.s + (size_t)(f0 + 64) * srow};
+    uint8_t *ssc = lds + 2 * GW_G * GW_SLOT;
+    const int npair = (int)srow / 8;
+    const int smask = (npair & (npair - 1)) ? 0 : min(npair - 1, 15);
+    {
+        /* LDS dword d of a half is dword c = d % sd of row d / sd, whose
+         * 8-byte piece c / 2 holds the step (c / 2) ^ (row & smask); wave w
+         * loads half w / 2, alternate instructions of the two waves */
+        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(wave < 2 ? sb[0] : sb[1], 64u * srow);
+        const uint32_t sd = srow / 4, inv = (1u << 20) / sd + 1;    /* exact for d < 64 sd, sd <= 64 */
+        uint8_t *dst = ssc + (wave >> 1) * 64 * srow;
+        for (uint32_t i = wave & 1; i < sd; i += 2) {
+            const uint32_t d = 64 * i + lane, row = (d * inv) >> 20, c = d - row * sd;
+            bdma4(rs, row * srow + 8 * ((c >> 1) ^ (row & (uint32_t)smask)) + 4 * (c & 1), 0, dst + 256 * i);
+        }
+    }
+    /* this wave's loads: token rows (rows past the tile's end answer with
+     * zeros) and weights; steps past the end read nothing but are counted */
+    const __amdgpu_buffer_rsrc_t rb = buf_rsrc(a.B, (uint32_t)a.nrows * (uint32_t)K * 2u);
+    const __amdgpu_buffer_rsrc_t rw[2] = {buf_rsrc(wb[0], 64u * rowb), buf_rsrc(wb[1], 64u * rowb)};
+    const __amdgpu_buffer_rsrc_t none = buf_rsrc(wb[0], 0);
+    uint32_t xofs[GW_XI];
+#pragma unroll
+    for (int i = 0; i < GW_XI; i++) {
+        const int t = 2 * (wave * GW_XI + i) + lane / 32;
+        const int src = t < ntok ? (a.row_tok ? a.row_tok[r0 + t] : r0 + t) : 0;
+        xofs[i] = t < ntok ? (uint32_t)src * (uint32_t)K * 2u + 16u * (uint32_t)swz_b(t, lane & 31) : OOB_OFFSET;
+    }
+    const uint32_t wofs0 = (uint32_t)(16 * wave + (lane & 14)) * rowb + 64u * (lane & 1) + 16u * gq;
+    const uint32_t wofs1 = wofs0 + rowb;
+    struct W { u32x4 v[GW_G][2][2]; };             /* [step][half][instruction] */
+    auto load = [&](W &w, int g, auto cpol) {
+        asm volatile("" ::: "memory");
+        uint8_t *slot = lds + (g & 1) * (GW_G * GW_SLOT);
+#pragma unroll
+        for (int k = 0; k < GW_G; k++)
+#pragma unroll
+            for (int i = 0; i < GW_XI; i++)
+                bdma16(g * GW_G + k < nst ? rb : none, xofs[i], (g * GW_G + k) * (KS * 2),
+                       slot + k * GW_SLOT + 1024 * (wave * GW_XI + i));
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int k = 0; k < GW_G; k++)
+                    w.v[k][m][j] = bload16<decltype(cpol)::value>(g * GW_G + k < nst ? rw[m] : none,
+                                                                  j ? wofs1 : wofs0, (g * GW_G + k) * (KS / 2));
+        asm volatile("" ::: "memory");
+    };
+    f4v acc[2] = {f4v{0.0f, 0.0f, 0.0f, 0.0f}, f4v{0.0f, 0.0f, 0.0f, 0.0f}};
+    const bool odd = lane & 1;
+    const uint8_t *sp = ssc + (16 * wave + rr) * srow;
+    const int sx = (16 * wave + rr) & smask;
+    auto compute = [&](const u32x4 (&v)[2][2], int g, int k) {
+        const int st = min(g * GW_G + k, nst - 1);  /* for the scales; the weights past the end are zeros */
+        const uint8_t *brow = lds + ((g & 1) * GW_G + k) * GW_SLOT + rr * (KS * 2);
+        float sc[2][2];
+        u32x4 op[2][2];                            /* [matrix half][128-index half of the step] */
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            const uint2 s8 = *(const uint2 *)(sp + m * 64 * srow + 8 * (st ^ sx));
+            /* as fp32 exponents: exact for the bytes 104..140 this path decodes */
+            sc[m][0] = __uint_as_float(((s8.x >> (8 * gq)) & 0xFFu) << 23);
+            sc[m][1] = __uint_as_float(((s8.y >> (8 * gq)) & 0xFFu) << 23);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t x0 = v[m][0][i], x1 = v[m][1][i];
+                const uint32_t p0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)x0, DPP_QUAD_1032, 0xF, 0xF, false);
+                const uint32_t p1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)x1, DPP_QUAD_1032, 0xF, 0xF, false);
+                op[m][0][i] = odd ? p1 : x0;       /* row 2 r + h: half 0, then half 1 */
+                op[m][1][i] = odd ? x1 : p0;
+            }
+        }
+        /* token operands one MFMA step ahead of their use */
+        h8 bop[2];
+        auto read_b = [&](int i) { return *(const h8 *)(brow + 16 * swz_b(rr, 16 * (i >> 2) + 4 * gq + (i & 3))); };
+        bop[0] = read_b(0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            if (i < 7) bop[(i + 1) & 1] = read_b(i + 1);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int m = 0; m < 2; m++)
+                acc[m] = mfma16(fp4_h8(op[m][i >> 2][i & 3], sc[m][i >> 2]), bop[i & 1], acc[m]);
+        }
+    };
+    auto run = [&](auto cpol) {
+        W ring[2];
+        load(ring[0], 0, cpol);
+        load(ring[1], 1, cpol);
+        for (int g = 0; g < ngr; g += 2) {
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                /* this group's tokens and weights (and, before the first, the
+                 * scales) have landed: only the next group's are outstanding */
+                __builtin_amdgcn_s_waitcnt(0x0F70 | GW_VM);
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int k = 0; k < GW_G; k++) {
+                    compute(ring[d].v[k], g + d, k);
+                    /* nothing of a later step moves up: its first use of a
+                     * weight register would wait for that register's load */
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                __builtin_amdgcn_s_waitcnt(0xC07F);    /* lgkmcnt(0): its slots have been read */
+                __builtin_amdgcn_s_barrier();
+                load(ring[d], g + d + 2, cpol);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    /* a bucket of one tile reads its weights once; with more, the tiles run
+     * side by side and the later ones find the weights in the L2 (non-temporal
+     * throughout: 1,000 tokens 1,267 against 1,100 us) */
+    if (tr.bucket <= 16) run(IC<CPOL_NT>{});
+    else run(IC<0>{});
+    __builtin_amdgcn_s_waitcnt(0x0F70);            /* the counted loads past the end */
+    bool scale_bad = false;                        /* this wave's 32 rows */
+    for (int m = 0; m < 2; m++)
+        for (int i = lane; i < 4 * (int)srow; i += 64)
+            scale_bad |= scales_bad(*(const uint32_t *)(ssc + (m * 64 + 16 * wave) * srow + 4 * i));
+    if (scale_bad) atomicOr(a.status, ST_SCALE_RANGE);
+
+    if (rr >= ntok) return;
+    unsigned range_bad = 0;
+    const size_t orow = (size_t)(r0 + rr) * N + f0 + 16 * wave + 4 * gq;
+    const int ex = b_row_exp(a, r0 + rr);
+    if constexpr (SWIGLU) {
+        *(uint2 *)((uint16_t *)a.out + orow) = swiglu_f16x4(acc[0], acc[1], ex, a.limit, range_bad);
+        if (range_bad) atomicOr(a.status, range_bad);
+    } else {
+        *(f4v *)((float *)a.out + orow) = unscale4(acc[0], ex);
+        *(f4v *)((float *)a.out + orow + 64) = unscale4(acc[1], ex);
+    }
+}
+
 /* ------------------------------------------------------------- combine --- */
 
 /* 4 consecutive outputs of one token per thread. The positions and weights
@@ -1325,7 +1556,7 @@ hipError_t to_f16_rows_launch(uint16_t *o, int *ex, const float *x, int rows, in
     return hipGetLastError();
 }
 
-int grouped_rows_per_tile(int tt) { return 16 * tt; }
+int grouped_rows_per_tile(int tt) { return tt == GROUPED_STREAM ? 16 : 16 * tt; }
 
 template <int WF, bool SW, int TT, int NS>
 static hipError_t grouped2_ns(const GroupedArgs &a, long items, hipStream_t st)
@@ -1393,9 +1624,34 @@ static hipError_t grouped3(const GroupedArgs &a, long items, hipStream_t st)
     return hipGetLastError();
 }
 
+template <bool SW>
+static hipError_t grouped_w(const GroupedArgs &a, long items, hipStream_t st)
+{
+    static bool attr_done = false;
+    if (!attr_done) {
+        const hipError_t e = hipFuncSetAttribute((const void *)k_grouped_w<SW>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, gw_lds(GW_KMAX));
+        if (e != hipSuccess) return e;
+        attr_done = true;
+    }
+    hipLaunchKernelGGL((k_grouped_w<SW>), dim3((unsigned)items), dim3(256), gw_lds(a.K), st, a);
+    return hipGetLastError();
+}
+
+bool grouped_stream_ok(long nrows, int K, int N)
+{
+    return K % KS == 0 && K <= GW_KMAX && N % 128 == 0 && (size_t)nrows * K * 2 < (1u << 31);
+}
+
 hipError_t grouped_launch(int fmt, bool swiglu, int tt, const GroupedArgs &a, long max_tiles,
                           hipStream_t st)
 {
+    if (tt == GROUPED_STREAM) {
+        if (fmt != FMT_FP4_E8M0 || !a.table || max_tiles <= 0 || a.nrows <= 0 || !grouped_stream_ok(a.nrows, a.K, a.N))
+            return hipErrorInvalidValue;
+        const long items = max_tiles * (a.N / (swiglu ? 64 : 128));
+        return swiglu ? grouped_w<true>(a, items, st) : grouped_w<false>(a, items, st);
+    }
     if (tt == 8) {
         /* 128-token tiles: FP4 only; byte offsets of every buffer fit 31 bits */
         const int feat = swiglu ? 128 : 256;

@@ -1473,10 +1473,23 @@ int dsv4_hip_gemm_mxfp8q_dev(void *C, int out_bf16, const uint8_t *Aq, const uin
 
 /* ------------------------------------------------------ grouped MoE --- */
 
-/* 16-row tiles when buckets are small (batched decode: few tokens per expert,
- * weight streaming dominates and occupancy matters), 128-row tiles otherwise
- * (prefill: weights are reused across a tile's rows). */
-static int grouped_tt(long pairs) { return pairs <= 4096 ? 1 : 8; }
+/* The form of the routed experts' GEMMs, by the mean bucket. Up to 28 rows an
+ * expert the weight stream is the bound: the 16-row tiles that stream to
+ * registers (4096 x 2048, 256 experts: 7 tokens 135 against 161 us of the
+ * LDS-staged 16-row tiles, 64 tokens 297 / 356, 701 tokens 870 / 1,005 and
+ * 1,128 of the 128-row tiles; at 33 rows an expert 1,233 / 1,374 / 1,193).
+ * With fewer than four steps of 256 to a row its setup costs more than it
+ * saves (inter 512: 62 against 59 us at 60 tokens): there the LDS-staged
+ * tiles, 16 rows up to 16 rows an expert, else 128 rows (weights reused
+ * across a tile; 64 experts, hidden 4096, inter 512: 60 tokens 89 against 101
+ * us, 300 tokens 146 / 134, 700 tokens 223 / 187). */
+static int grouped_tt(long pairs, int n_experts, int n, int hidden, int inter)
+{
+    if (pairs <= 28L * n_experts && hidden >= 1024 && inter >= 1024 && grouped_stream_ok(n, hidden, inter) &&
+        grouped_stream_ok(pairs, inter, hidden))
+        return GROUPED_STREAM;
+    return pairs <= 16L * n_experts ? 1 : 8;
+}
 
 static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4ExpertW *table,
                         int n_experts, const int *idx, const float *w, int topk,
@@ -1484,7 +1497,7 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
                         int inter, float limit, hipStream_t st)
 {
     const long P = (long)n * topk;
-    int tt = grouped_tt(P);
+    int tt = grouped_tt(P, n_experts, n, hidden, inter);
     /* the 128-row kernel takes 256 down rows per workgroup and 31-bit offsets */
     if (tt == 8 && (hidden % 256 || (size_t)P * inter * 2 >= (1u << 31) ||
                     (size_t)n * hidden * 2 >= (1u << 31) || (size_t)inter * hidden / 2 >= (1u << 31)))
@@ -1492,8 +1505,8 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     const int trows = grouped_rows_per_tile(tt);
     size_t off = 0;
     auto take = [&](size_t b) { const size_t o = off; off += (b + 255) & ~(size_t)255; return o; };
-    /* every bucket adds at most one partial tile */
-    const long max_tiles = (P + trows - 1) / trows + n_experts;
+    /* every bucket adds at most one partial tile, and every tile has a row */
+    const long max_tiles = std::min(P, (P + trows - 1) / trows + n_experts);
     const size_t o_grp = take((size_t)(n_experts + 1) * 4), o_tp = take((size_t)(n_experts + 1) * 4);
     const size_t o_tg = take((size_t)(max_tiles + 4) * sizeof(TileRec));
     const size_t o_pos = take((size_t)P * 4), o_row = take((size_t)P * 4);

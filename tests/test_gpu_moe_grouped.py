@@ -459,3 +459,78 @@ def _torch_all_tokens_exact(lib, arena, keep, x, idx, w, got, n, H, I, topk, lim
     den = np.sqrt(np.sum(ref ** 2, axis=1))
     r = num / den
     assert np.all(r <= REL_L2_TOL), f"{int(np.sum(r > REL_L2_TOL))} tokens beyond 1e-3, worst {float(r.max()):.3e}"
+
+
+def bucket_case(lib, pkg, counts, hidden, inter, seed):
+    """One expert per token, expert e chosen by counts[e] tokens."""
+    gen = torch.Generator().manual_seed(seed)
+    dgen = torch.Generator(device=DEV).manual_seed(seed)
+    ids = np.concatenate([np.full(c, e, np.int32) for e, c in enumerate(counts)])
+    np.random.default_rng(seed).shuffle(ids)
+    n = len(ids)
+    experts = [DevExpert(lib, pkg, "fp4", inter, hidden, dgen) for _ in counts]
+    return experts, bf16_rows(gen, n, hidden), ids.reshape(n, 1), np.ones((n, 1), np.float32)
+
+
+@pytest.mark.parametrize("counts,hidden,inter", [
+    ([1, 16, 17, 15, 0, 2, 33], 1024, 1024),     # tiles of one bucket, several, a last one of one row
+    ([3, 0, 20], 1280, 1024),                    # 5 steps (an odd group), scale rows of 5 pieces
+    ([2, 5], 1024, 1792),                        # 7 steps down
+    ([1], 8192, 1024),                           # the widest rows, one tile in all
+    ([28, 28], 2048, 1024),                      # the last mean bucket of the streaming form
+])
+def test_grouped_stream_tiles(lib, pkg, oracle, counts, hidden, inter):
+    """Up to 28 rows an expert, hidden and inter from 1024: the weights stream
+    to registers (k_grouped_w). Every token against the oracle, two calls
+    bit-identical."""
+    experts, x, idx, w = bucket_case(lib, pkg, counts, hidden, inter, 77 + hidden + inter + len(counts))
+    lib.status()
+    got = run_dev(lib, experts, None, x, idx, w, hidden, inter)
+    again = run_dev(lib, experts, None, x, idx, w, hidden, inter)
+    assert lib.status() == 0
+    assert np.array_equal(bits(got), bits(again))
+    want = oracle_tokens(oracle, experts, None, x, idx, w, list(range(len(x))))
+    e = rel_l2(got, want)
+    assert e <= REL_L2_TOL, f"rel L2 {e:.3e} (max abs {max_abs(got, want):.3e})"
+
+
+@pytest.mark.parametrize("mat,at", [(0, 5), (1, 1024 * 32 - 1), (2, 1024 * 16 + 3)])
+def test_grouped_stream_scale_range_flag(lib, pkg, mat, at):
+    """A scale byte outside 104..140 in any matrix raises status bit 2, an
+    unused expert's does not."""
+    experts, x, idx, w = bucket_case(lib, pkg, [3, 0, 2], 1024, 1024, 5)
+    lib.status()
+    experts[1].m[mat].S[at] = 141
+    torch.cuda.synchronize()
+    run_dev(lib, experts, None, x, idx, w, 1024, 1024)
+    assert lib.status() == 0
+    experts[2].m[mat].S[at] = 103
+    torch.cuda.synchronize()
+    run_dev(lib, experts, None, x, idx, w, 1024, 1024)
+    assert lib.status() == 4
+
+
+@pytest.mark.parametrize("counts,hidden,inter", [
+    ([3, 0, 18], 1024, 1024),                    # streaming tiles
+    ([3, 18], 512, 512),                         # LDS-staged 16-row tiles
+    ([40, 30], 512, 512),                        # 128-row tiles
+])
+def test_grouped_dword_aligned_experts(lib, pkg, oracle, counts, hidden, inter):
+    """Expert weights and scales that start on a 4-byte boundary only."""
+    experts, x, idx, w = bucket_case(lib, pkg, counts, hidden, inter, 91 + hidden)
+    keep = []
+    for e in experts:
+        for m, name in zip(e.m, ("w1", "w3", "w2")):
+            q = getattr(e.desc, name)
+            for field, t in (("w", m.W), ("s", m.S)):
+                buf = torch.empty(t.numel() + 4, dtype=torch.uint8, device=DEV)
+                buf[4:] = t
+                keep.append(buf)
+                setattr(q, field, buf.data_ptr() + 4)
+    torch.cuda.synchronize()
+    lib.status()
+    got = run_dev(lib, experts, None, x, idx, w, hidden, inter)
+    assert lib.status() == 0
+    want = oracle_tokens(oracle, experts, None, x, idx, w, list(range(len(x))))
+    e = rel_l2(got, want)
+    assert e <= REL_L2_TOL, f"rel L2 {e:.3e} (max abs {max_abs(got, want):.3e})"
