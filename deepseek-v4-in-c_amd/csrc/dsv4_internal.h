@@ -333,6 +333,15 @@ struct SeamGemmArgs {
 bool gemm_seam_ok(int M, int N, int K);
 hipError_t gemm_seam_launch(const SeamGemmArgs &s, bool w_f32s, hipStream_t st);
 
+/* The same GEMMs in tiles of 64 features x 16 nt tokens (dsv4_gemm_thin.hip);
+ * gemm_thin_nt / gemm_thin_seam_nt: the nt a shape takes, 0 for the large
+ * tiles. */
+int gemm_thin_nt(int M, int N, int K);
+int gemm_thin_seam_nt(int M, int N, int K);
+hipError_t gemm_thin_fp8_launch(const GemmArgs &g, bool w_f32s, bool out_bf16, int nt, hipStream_t st);
+hipError_t gemm_thin_mx_launch(const GemmArgs &g, bool out_bf16, int nt, hipStream_t st);
+hipError_t gemm_thin_seam_launch(const SeamGemmArgs &s, bool w_f32s, int nt, hipStream_t st);
+
 /* ---------------------------------------------- dequant / quantizers --- */
 hipError_t dequant_launch(int fmt, const DSV4QMat &m, float *out, hipStream_t st);
 hipError_t quant_fp4_mx_launch(uint8_t *W, uint8_t *S, const float *w, int rows,

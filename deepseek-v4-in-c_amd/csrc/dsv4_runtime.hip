@@ -686,14 +686,16 @@ void *dsv4_hip_device_ptr(const void *p)
  * every nt. From MMQ_MFMA_MIN_TOKENS tokens on, packed matrices the grouped
  * kernel takes (rows, cols multiples of 128; FP8 with 128x128 blocks or FP4
  * with 1x32) run as one dense fp16-MFMA GEMM (x row-scaled by a power of two
- * and rounded to fp16, weights decoded exactly, fp32 accumulation): FP8 from
- * MMQ_SEAM_GEMM_MIN_TOKENS tokens on in the GEMM-shaped seam kernel (128 x
- * 256 tiles), else in the grouped kernel with one group (the same bits);
- * fewer tokens run the block-scaled MFMA GEMV where its geometry fits, else
- * the per-token VALU GEMV. The seam kernel's tiles fill the device only
- * from about 2048 tokens (4096 x 4096 FP8: 64 us from 128 to 1024 tokens,
- * 79 us at 2048), the grouped form's 64-token tiles from far fewer (32 us
- * at 128, 59 us at 1024, 82 us at 1536): the switch sits between. */
+ * and rounded to fp16, weights decoded exactly, fp32 accumulation): FP8 in
+ * tiles of 64 rows x 16 or 32 tokens while those are few enough
+ * (gemm_thin_seam_nt), from MMQ_SEAM_GEMM_MIN_TOKENS tokens on in the
+ * GEMM-shaped seam kernel (128 x 256 tiles), else in the grouped kernel with
+ * one group (the same bits in all three); fewer tokens run the block-scaled
+ * MFMA GEMV where its geometry fits, else the per-token VALU GEMV. The seam
+ * kernel's tiles fill the device only from about 2048 tokens (4096 x 4096
+ * FP8: 64 us from 128 to 1024 tokens, 79 us at 2048), the grouped form's
+ * 64-token tiles from far fewer (59 us at 1024, 82 us at 1536): the switch
+ * sits between. */
 constexpr int MMQ_MFMA_MIN_TOKENS = 32;
 constexpr int MMQ_SEAM_GEMM_MIN_TOKENS = 1280;
 /* From this many tokens the block-scaled MFMA GEMV splits x once into its
@@ -728,6 +730,13 @@ static int enqueue_mmq(const DSV4QMat &d, int fmt, const float *x, float *y, int
         uint16_t *x16 = (uint16_t *)g.x16.p;
         int *ex = (int *)((uint8_t *)g.x16.p + xb);
         HIPCHK(to_f16_rows_launch(x16, ex, x, nt, d.cols, st), "x fp16 launch");
+        if (const int tn = fmt != FMT_FP4_E8M0 && aligned16(d.w) ? gemm_thin_seam_nt(nt, d.rows, d.cols) : 0) {
+            SeamGemmArgs sg;
+            sg.X = x16; sg.ex = ex; sg.W = (const uint8_t *)d.w; sg.Sw = d.s; sg.C = y;
+            sg.M = nt; sg.N = d.rows; sg.K = d.cols;
+            HIPCHK(gemm_thin_seam_launch(sg, fmt == FMT_FP8_F32S, tn, st), "seam GEMM launch");
+            return 0;
+        }
         if (fmt != FMT_FP4_E8M0 && nt >= MMQ_SEAM_GEMM_MIN_TOKENS && aligned16(d.w) &&
             gemm_seam_ok(nt, d.rows, d.cols)) {
             SeamGemmArgs sg;

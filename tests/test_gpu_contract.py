@@ -361,6 +361,31 @@ def test_seam_gemm_bits_equal_grouped_form(lib, pkg, oracle, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["fp8", "fp8f"])
+@pytest.mark.parametrize("rows,cols", [(2048, 128), (2176, 640), (2048, 1152)])
+def test_seam_tile_sizes_same_bits(lib, pkg, oracle, rows, cols, fmt):
+    """The three forms of the FP8 seam give a token the same bits: 16- and
+    32-token tiles of 64 features (both edges of each, a part of a group of
+    reduction blocks, feature tiles no multiple of eight), the grouped form
+    above them and the 128 x 256 tiles from 1280 tokens."""
+    rng = np.random.default_rng(rows + cols + len(fmt))
+    m, want_of = _fp8_resident(lib, pkg, oracle, fmt, rng, rows, cols)
+    nt = 1290
+    x = rng.standard_normal((nt, cols)).astype(np.float32)
+    x[0] *= 1e5
+    x[1] *= 1e-9
+    x[2] = 0.0
+    x = np.ascontiguousarray(x)
+    got = {n: lib.mmq_n(m.desc, np.ascontiguousarray(x[:n].reshape(-1)), n).reshape(n, rows)
+           for n in (32, 33, 128, 129, 147, 300, 400, 1279, nt)}
+    want = want_of(np.ascontiguousarray(x[:33].reshape(-1)), 33).reshape(33, rows)
+    for t in range(33):
+        assert rel_l2(got[33][t], want[t]) <= REL_L2_TOL, t
+    for n, y in got.items():
+        assert np.array_equal(bits(y), bits(got[nt][:n])), n
+    m.drop()
+
+
+@pytest.mark.parametrize("fmt", ["fp8", "fp8f"])
 def test_fp8_16_token_tiles_ring_depths(lib, pkg, oracle, fmt):
     """FP8 weights, 32-192 tokens: 16-token tiles with a two-stage ring when
     the grid outnumbers the CUs (150 tokens x 4096 rows: 320 workgroups),

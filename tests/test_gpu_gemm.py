@@ -195,6 +195,47 @@ def test_gemm_prequantized_matches_fused(lib, pkg, oracle):
     assert np.array_equal(bits(C.cpu().numpy()), bits(fused))
 
 
+@pytest.mark.parametrize("n,k,big", [(1024, 128, 1040), (1024, 1152, 1040), (384, 640, 2740),
+                                     (2048, 8192, 520)])
+@pytest.mark.parametrize("form", ["fp8f", "fp8", "mx"])
+def test_gemm_tile_sizes_same_bits(lib, pkg, oracle, n, k, big, form):
+    """A token's outputs have the same bits from the 64-feature tiles of 16,
+    32 and 64 tokens (the edges of a tile and of each tile size's range, one
+    block to 64 of the reduction, feature tiles no multiple of eight) as from
+    the 128 x 256 ones, which `big` tokens take; fp32 and bf16 results, and
+    quantized operands as their entry points take them."""
+    rng = np.random.default_rng(n + k + len(form))
+    A = rng.standard_normal((big, k)).astype(np.float32)
+    W, S = make_weight(oracle, rng, n, k, f32s=form == "fp8f")
+    if form == "mx":
+        run = lambda a, ob: run_gemm_mx(lib, pkg, a, W, S, n, k, ob, 0)
+    else:
+        run = lambda a, ob: run_gemm(lib, pkg, a, W, S, n, k, form == "fp8f", ob, 0)
+    want = run(A, 0)
+    want_bf16 = run(A, 1)
+    tiles = n // 64
+    edges = {16 * nt * (256 // tiles) for nt in (1, 2, 4)}
+    for m in sorted({1, 15, 16, 17, 33, 65} | edges | {e + 1 for e in edges}):
+        m = min(m, big)
+        assert np.array_equal(bits(run(A[:m], 0)), bits(want[:m])), m
+        assert np.array_equal(run(A[:m], 1), want_bf16[:m]), m
+    m = 37
+    dW, dS = dev(W), dev(S)
+    desc = pkg.qmat(pkg.DSV4_WFP8_F32S if form == "fp8f" else pkg.DSV4_WFP8, dW.data_ptr(), dS.data_ptr(),
+                    n, k, 128, 128)
+    C = torch.empty((m, n), dtype=torch.float32, device=DEV)
+    if form == "mx":
+        Q, Sa = oracle.quant_act_mxfp8(A[:m])
+        dQ, dSa = dev(Q), dev(Sa)
+        lib.gemm_mxfp8q_dev(C.data_ptr(), 0, dQ.data_ptr(), dSa.data_ptr(), m, desc)
+    else:
+        Q, Sa = oracle.quant_act_fp8_1x128(A[:m])
+        dQ, dSa = dev(Q), dev(np.ascontiguousarray(Sa.reshape(m, k // 128).T))
+        lib.gemm_fp8q_dev(C.data_ptr(), 0, dQ.data_ptr(), dSa.data_ptr(), m, desc)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(C.cpu().numpy()), bits(want[:m]))
+
+
 def test_gemm_deterministic(lib, pkg, oracle):
     rng = np.random.default_rng(9)
     m, n, k = 256, 512, 512
