@@ -3,14 +3,12 @@
  * shapes whose 128 x 256 tiles leave most of the device idle: few tokens, or
  * a matrix of few rows.
  *
- * Three forms of C[m][n] = sum_k A[m][k] W[n][k], each with the products, the
+ * Two forms of C[m][n] = sum_k A[m][k] W[n][k], each with the products, the
  * reduction order and so the bits of its large-tile kernel:
  *   T_FP8   e4m3 tokens with fp32 1 x 128 scales, fp32 or E8M0 weight blocks,
  *           every 128-wide block's product folded into fp32 (k_gemm_fp8)
  *   T_MX    MXFP8 tokens, E8M0 weight blocks, both in the MFMA's scale
  *           operands (k_gemm_mx)
- *   T_SEAM  fp16 tokens scaled by 2^ex, e4m3 weights decoded to fp16 in
- *           registers, block partials folded into fp32 (k_gemm_seam)
  *
  * SCHEDULE
  *   A workgroup of four waves owns 64 features x 16 NT tokens; wave w the 16
@@ -39,10 +37,9 @@ namespace {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) void lds_void;
 
-enum { T_FP8 = 0, T_MX = 1, T_SEAM = 2 };
+enum { T_FP8 = 0, T_MX = 1 };
 
 constexpr int TB = 128;                            /* reduction block           */
 constexpr int TG = 4;                              /* blocks per group, a wave each */
@@ -51,13 +48,11 @@ constexpr int T_KMAX = 64 * TB;
 constexpr uint32_t T_OOB = 0x80000000u;            /* beyond every buffer       */
 constexpr int T_E8M0_ONE = 127;
 
-template <int MODE, int NT> struct Thin {
-    static constexpr int XROW = MODE == T_SEAM ? 2 * TB : TB;      /* token bytes per block   */
-    static constexpr int XI = 16 * NT * XROW / 1024;               /* token loads per block   */
-    static constexpr int SI = MODE == T_SEAM ? 0 : 1;              /* token scale loads       */
-    static constexpr int XBLK = 1024 * XI + 256 * SI;              /* LDS of a block          */
+template <int NT> struct Thin {
+    static constexpr int XI = 16 * NT * TB / 1024;                 /* token loads per block   */
+    static constexpr int XBLK = 1024 * XI + 256;                   /* LDS of a block          */
     static constexpr int LDS = 2 * TG * XBLK;
-    static constexpr int VM = 2 * TG + XI + SI;                    /* a wave's loads a group  */
+    static constexpr int VM = 2 * TG + XI + 1;                     /* a wave's loads a group  */
     static_assert(VM <= 63, "vmcnt range");
 };
 
@@ -86,24 +81,12 @@ __device__ __forceinline__ uint32_t t_bf16(float f)
     return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 
-/* eight e4m3 to eight fp16, exact */
-__device__ __forceinline__ h8v t_f16(uint32_t d0, uint32_t d1)
-{
-    u32x4 v;
-    v.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d0, 1.0f, false));
-    v.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d0, 1.0f, true));
-    v.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d1, 1.0f, false));
-    v.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d1, 1.0f, true));
-    return __builtin_bit_cast(h8v, v);
-}
-
 } // namespace
 
 /* one call's operands in any of the forms */
 struct ThinArgs {
-    const void *A;            /* tokens [M][K]: e4m3, or fp16 (T_SEAM)            */
+    const void *A;            /* e4m3 tokens [M][K]                               */
     const void *Sa;           /* token scales (a dword per token and block)       */
-    const int *ex;            /* T_SEAM: the power of two of each token           */
     const uint8_t *W;
     const void *Sw;
     void *C;
@@ -114,7 +97,7 @@ struct ThinArgs {
 template <int MODE, bool WF32S, bool OUT_BF16, int NT>
 __global__ __launch_bounds__(256) void k_gemm_thin(ThinArgs a)
 {
-    using C = Thin<MODE, NT>;
+    using C = Thin<NT>;
     extern __shared__ __align__(16) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = wave_in_group();
     const int rr = lane & 15, gq = lane >> 4;
@@ -127,20 +110,18 @@ __global__ __launch_bounds__(256) void k_gemm_thin(ThinArgs a)
     const int n0 = lin / mt * TN, m0 = lin % mt * (16 * NT);
     const int nkb = a.K / TB, ngr = (nkb + 2 * TG - 1) / (2 * TG) * 2;
 
-    const uint32_t xld = (uint32_t)a.K * (MODE == T_SEAM ? 2u : 1u);
-    const __amdgpu_buffer_rsrc_t rx = t_rsrc(a.A, (uint32_t)a.M * xld);
+    const __amdgpu_buffer_rsrc_t rx = t_rsrc(a.A, (uint32_t)a.M * (uint32_t)a.K);
     const __amdgpu_buffer_rsrc_t rw = t_rsrc(a.W + (size_t)n0 * a.K, (uint32_t)TN * (uint32_t)a.K);
     const __amdgpu_buffer_rsrc_t none = t_rsrc(a.W, 0);
-    const __amdgpu_buffer_rsrc_t rs = t_rsrc(MODE == T_SEAM ? a.W : a.Sa, MODE == T_SEAM ? 0u :
-        4u * ((uint32_t)(nkb - 1) * (uint32_t)a.sa_kb + (uint32_t)(a.M - 1) * (uint32_t)a.sa_tok + 1u));
+    const __amdgpu_buffer_rsrc_t rs = t_rsrc(
+        a.Sa, 4u * ((uint32_t)(nkb - 1) * (uint32_t)a.sa_kb + (uint32_t)(a.M - 1) * (uint32_t)a.sa_tok + 1u));
     /* token row r of a block holds chunk c at slot swx(r, c) */
-    auto swx = [](int r, int c) { return MODE == T_SEAM ? c ^ (r & 15) : c ^ ((r >> 1) & 7); };
+    auto swx = [](int r, int c) { return c ^ ((r >> 1) & 7); };
     uint32_t xofs[C::XI];
 #pragma unroll
     for (int i = 0; i < C::XI; i++) {
-        constexpr int CPR = C::XROW / 16, RPI = 64 / CPR;          /* chunks per row, rows per load */
-        const int r = RPI * i + lane / CPR, c = swx(r, lane % CPR);
-        xofs[i] = m0 + r < a.M ? (uint32_t)(m0 + r) * xld + 16u * (uint32_t)c : T_OOB;
+        const int r = 8 * i + lane / 8, c = swx(r, lane & 7);
+        xofs[i] = m0 + r < a.M ? (uint32_t)(m0 + r) * (uint32_t)a.K + 16u * (uint32_t)c : T_OOB;
     }
     const int mlane = m0 + (lane & (16 * NT - 1));
     const uint32_t sofs = lane < 16 * NT && mlane < a.M ? 4u * (uint32_t)mlane * (uint32_t)a.sa_tok : T_OOB;
@@ -156,8 +137,8 @@ __global__ __launch_bounds__(256) void k_gemm_thin(ThinArgs a)
         uint8_t *dst = lds + ((g & 1) * TG + wave) * C::XBLK;
 #pragma unroll
         for (int i = 0; i < C::XI; i++)
-            t_dma16(kb < nkb ? rx : none, xofs[i], kb * C::XROW, dst + 1024 * i);
-        if constexpr (C::SI) t_dma4(kb < nkb ? rs : none, sofs, 4 * kb * a.sa_kb, dst + 1024 * C::XI);
+            t_dma16(kb < nkb ? rx : none, xofs[i], kb * TB, dst + 1024 * i);
+        t_dma4(kb < nkb ? rs : none, sofs, 4 * kb * a.sa_kb, dst + 1024 * C::XI);
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
@@ -195,52 +176,33 @@ __global__ __launch_bounds__(256) void k_gemm_thin(ThinArgs a)
         }
         const uint32_t sw = (uint32_t)__builtin_amdgcn_readlane((int)wsc, min(kb, nkb - 1));
         const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        if constexpr (MODE == T_SEAM) {
-            v4f part[NT];
+        v8i w;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const u32x4 &h = j < 2 ? lo : hi;
-                const h8v av = (j & 1) ? t_f16(h.z, h.w) : t_f16(h.x, h.y);
+        for (int e = 0; e < 4; e++) {
+            w[e] = (int)lo[e];
+            w[4 + e] = (int)hi[e];
+        }
 #pragma unroll
-                for (int u = 0; u < NT; u++) {
-                    const int t = 16 * u + rr;
-                    const h8v b = *(const h8v *)(blk + t * C::XROW + 16 * swx(t, 8 * (j >> 1) + 2 * gq + (j & 1)));
-                    part[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b, j == 0 ? zero : part[u], 0, 0, 0);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < NT; u++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[u][e] = fmaf(part[u][e], __uint_as_float(sw), acc[u][e]);
-        } else {
-            v8i w;
+        for (int u = 0; u < NT; u++) {
+            const int t = 16 * u + rr;
+            const u32x4 b0 = *(const u32x4 *)(blk + t * TB + 16 * swx(t, gq));
+            const u32x4 b1 = *(const u32x4 *)(blk + t * TB + 16 * swx(t, gq + 4));
+            const uint32_t ts = *(const uint32_t *)(blk + 1024 * C::XI + 4 * t);
+            v8i b;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                w[e] = (int)lo[e];
-                w[4 + e] = (int)hi[e];
+                b[e] = (int)b0[e];
+                b[4 + e] = (int)b1[e];
             }
+            if constexpr (MODE == T_MX) {
+                acc[u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, b, acc[u], 0, 0, 0, (int)sw, 0,
+                                                                         (int)((ts >> (8 * gq)) & 0xFFu));
+            } else {
+                const v4f p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, b, zero, 0, 0, 0, T_E8M0_ONE,
+                                                                              0, T_E8M0_ONE);
+                const float cs = __uint_as_float(ts) * __uint_as_float(sw);
 #pragma unroll
-            for (int u = 0; u < NT; u++) {
-                const int t = 16 * u + rr;
-                const u32x4 b0 = *(const u32x4 *)(blk + t * TB + 16 * swx(t, gq));
-                const u32x4 b1 = *(const u32x4 *)(blk + t * TB + 16 * swx(t, gq + 4));
-                const uint32_t ts = *(const uint32_t *)(blk + 1024 * C::XI + 4 * t);
-                v8i b;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    b[e] = (int)b0[e];
-                    b[4 + e] = (int)b1[e];
-                }
-                if constexpr (MODE == T_MX) {
-                    acc[u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, b, acc[u], 0, 0, 0, (int)sw, 0,
-                                                                             (int)((ts >> (8 * gq)) & 0xFFu));
-                } else {
-                    const v4f p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w, b, zero, 0, 0, 0, T_E8M0_ONE,
-                                                                                  0, T_E8M0_ONE);
-                    const float cs = __uint_as_float(ts) * __uint_as_float(sw);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) acc[u][e] = fmaf(p[e], cs, acc[u][e]);
-                }
+                for (int e = 0; e < 4; e++) acc[u][e] = fmaf(p[e], cs, acc[u][e]);
             }
         }
     };
@@ -269,12 +231,7 @@ __global__ __launch_bounds__(256) void k_gemm_thin(ThinArgs a)
         const int m = m0 + 16 * u + rr;
         if (m >= a.M) continue;
         const size_t o = (size_t)m * a.N + n0 + 16 * wave + 4 * gq;
-        v4f v = acc[u];
-        if constexpr (MODE == T_SEAM) {
-            const int ex = a.ex[m];
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = ex == 0 ? v[e] : ldexpf(v[e], -ex);
-        }
+        const v4f v = acc[u];
         if constexpr (OUT_BF16) {
             uint2 pk;
             pk.x = t_bf16(v[0]) | (t_bf16(v[1]) << 16);
@@ -289,7 +246,7 @@ __global__ __launch_bounds__(256) void k_gemm_thin(ThinArgs a)
 template <int MODE, bool WS, bool OB, int NT>
 static hipError_t thin_launch(const ThinArgs &a, hipStream_t st)
 {
-    using C = Thin<MODE, NT>;
+    using C = Thin<NT>;
     static bool attr_done = false;
     if (!attr_done) {
         const hipError_t e = hipFuncSetAttribute((const void *)k_gemm_thin<MODE, WS, OB, NT>,
@@ -304,10 +261,10 @@ static hipError_t thin_launch(const ThinArgs &a, hipStream_t st)
 
 /* the loads address A, W and Sa with 31-bit byte offsets, and a row block's
  * scales fit one register */
-static bool thin_ok(int M, int N, int K, size_t a_row_bytes, size_t sa_dwords)
+static bool thin_ok(int M, int N, int K)
 {
-    return M > 0 && N % 128 == 0 && K % TB == 0 && K <= T_KMAX && (size_t)M * a_row_bytes < (1u << 31) &&
-           sa_dwords < (1u << 29) && (size_t)M * N / 1024 < (1u << 31);
+    return M > 0 && N % 128 == 0 && K % TB == 0 && K <= T_KMAX && (size_t)M * K < (1u << 31) &&
+           (size_t)M * N / 1024 < (1u << 31);
 }
 
 template <int MODE, bool WS>
@@ -323,7 +280,7 @@ static hipError_t thin_nt(const ThinArgs &a, bool out_bf16, int nt, hipStream_t 
 static ThinArgs thin_args(const GemmArgs &g)
 {
     ThinArgs a;
-    a.A = g.Aq; a.Sa = g.Sa; a.ex = nullptr; a.W = g.W; a.Sw = g.Sw; a.C = g.C;
+    a.A = g.Aq; a.Sa = g.Sa; a.W = g.W; a.Sw = g.Sw; a.C = g.C;
     a.M = g.M; a.N = g.N; a.K = g.K; a.sa_tok = g.sa_tok; a.sa_kb = g.sa_kb;
     return a;
 }
@@ -339,15 +296,6 @@ hipError_t gemm_thin_mx_launch(const GemmArgs &g, bool out_bf16, int nt, hipStre
     return thin_nt<T_MX, false>(thin_args(g), out_bf16, nt, st);
 }
 
-hipError_t gemm_thin_seam_launch(const SeamGemmArgs &s, bool w_f32s, int nt, hipStream_t st)
-{
-    ThinArgs a;
-    a.A = s.X; a.Sa = nullptr; a.ex = s.ex; a.W = s.W; a.Sw = s.Sw; a.C = s.C;
-    a.M = s.M; a.N = s.N; a.K = s.K; a.sa_tok = 0; a.sa_kb = 0;
-    if (nt == 1) return w_f32s ? thin_launch<T_SEAM, true, false, 1>(a, st) : thin_launch<T_SEAM, false, false, 1>(a, st);
-    return w_f32s ? thin_launch<T_SEAM, true, false, 2>(a, st) : thin_launch<T_SEAM, false, false, 2>(a, st);
-}
-
 /* workgroups of nt 16-token groups a tile */
 static long thin_wgs(int M, int N, int nt) { return ((long)M + 16 * nt - 1) / (16 * nt) * (N / TN); }
 
@@ -360,23 +308,10 @@ static long thin_wgs(int M, int N, int nt) { return ((long)M + 16 * nt - 1) / (1
  * token tile, through registers. */
 int gemm_thin_nt(int M, int N, int K)
 {
-    if (!thin_ok(M, N, K, (size_t)K, (size_t)M * K / TB)) return 0;
+    if (!thin_ok(M, N, K)) return 0;
     for (int nt = 1; nt <= 4; nt *= 2)
         if (thin_wgs(M, N, nt) <= 256) return nt;
     return 0;
-}
-
-/* Against the grouped form (us of the call, conversion included): 1024 x 4096
- * 32 tokens 14.7 / 22.5, 128 tokens 15.8 / 23.7, 333 tokens (nt 2) 21.5 /
- * 38.0, 700 tokens (nt 2, 352 workgroups) 32.9 / 40.8; 4096 x 4096 32 tokens
- * 15.0 / 23.6, 77 tokens (nt 2) 18.5 / 24.1, 128 tokens 19.1 / 24.9; beyond,
- * the grouped form (32768 x 1024, 32 tokens, 512 workgroups 14.0 / 13.5; 4096
- * x 4096, 333 tokens, 704 workgroups 40.9 / 37.9). */
-int gemm_thin_seam_nt(int M, int N, int K)
-{
-    if (!thin_ok(M, N, K, 2 * (size_t)K, 0)) return 0;
-    if (thin_wgs(M, N, 1) <= 256) return 1;
-    return thin_wgs(M, N, 2) <= 384 ? 2 : 0;
 }
 
 } // namespace dsv4

@@ -333,14 +333,12 @@ struct SeamGemmArgs {
 bool gemm_seam_ok(int M, int N, int K);
 hipError_t gemm_seam_launch(const SeamGemmArgs &s, bool w_f32s, hipStream_t st);
 
-/* The same GEMMs in tiles of 64 features x 16 nt tokens (dsv4_gemm_thin.hip);
- * gemm_thin_nt / gemm_thin_seam_nt: the nt a shape takes, 0 for the large
+/* The FP8 and MXFP8 GEMMs in tiles of 64 features x 16 nt tokens
+ * (dsv4_gemm_thin.hip); gemm_thin_nt: the nt a shape takes, 0 for the large
  * tiles. */
 int gemm_thin_nt(int M, int N, int K);
-int gemm_thin_seam_nt(int M, int N, int K);
 hipError_t gemm_thin_fp8_launch(const GemmArgs &g, bool w_f32s, bool out_bf16, int nt, hipStream_t st);
 hipError_t gemm_thin_mx_launch(const GemmArgs &g, bool out_bf16, int nt, hipStream_t st);
-hipError_t gemm_thin_seam_launch(const SeamGemmArgs &s, bool w_f32s, int nt, hipStream_t st);
 
 /* ---------------------------------------------- dequant / quantizers --- */
 hipError_t dequant_launch(int fmt, const DSV4QMat &m, float *out, hipStream_t st);
@@ -465,11 +463,16 @@ struct GroupedArgs {
     float limit;
     unsigned *status;
 };
-/* tt: 1 or 4 (16- or 64-row tiles), 8 (128-row, FP4) or GROUPED_STREAM
- * (16-row, FP4 experts of a table, geometry as grouped_stream_ok) */
-constexpr int GROUPED_STREAM = 5;
+/* tt: 1 or 4 (16- or 64-row tiles), 8 (128-row, FP4), GROUPED_STREAM (16-row,
+ * FP4 experts of a table, geometry as grouped_stream_ok) or GROUPED_DENSE (one
+ * FP8 matrix, operands as grouped_dense_cost) */
+constexpr int GROUPED_STREAM = 5, GROUPED_DENSE = 6;
 int grouped_rows_per_tile(int tt);
 bool grouped_stream_ok(long nrows, int K, int N);
+/* the cost of the GROUPED_DENSE form, in the units of GROUPED_DENSE_SEAM per
+ * round of 256 workgroups of the seam GEMM; 0: it does not take the operands */
+constexpr long GROUPED_DENSE_SEAM = 60;
+long grouped_dense_cost(const GroupedArgs &a, int fmt, bool swiglu);
 hipError_t grouped_launch(int fmt, bool swiglu, int tt, const GroupedArgs &a, long max_tiles,
                           hipStream_t st);
 

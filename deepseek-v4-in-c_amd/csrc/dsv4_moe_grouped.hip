@@ -1482,6 +1482,199 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     }
 }
 
+/* ------------------------------------------------ dense FP8 (many tokens) --- */
+
+/* One FP8 matrix (or the shared expert's w1 and w3) against many tokens: the
+ * dense form in tiles of 128 weight rows x 16 T tokens. Products, order and
+ * so bits are k_grouped2's.
+ *
+ * Eight waves, 4 x 32 rows (gate/up: 16 w1 rows and the w3 rows of the same
+ * features) by 2 x 8 T tokens (T = 4, 6) or four by 16 T (T = 1 .. 3). A stage is one 128-wide reduction block, rows
+ * and tokens by buffer loads straight to LDS, NST stages in a ring. A wave
+ * reads its operands of the next stage while it multiplies one, a read to
+ * two MFMAs and a load between them, so that the barrier between stages waits
+ * for no read. A row block's scales sit in one register, one block per lane.
+ *
+ * Bound: the LDS path of a wave (32 clk per 16-byte read, 16 clk per MFMA; no
+ * reads: 6 of 19 us gone at 4096 x 4096, 333 tokens, T = 3) and the loads' L2
+ * traffic (no loads: 5). Reads and MFMAs of one wave hardly overlap, so waves
+ * per SIMD count: T = 6 30.6 us in eight waves, 37.7 in four. 4096 x 4096, the
+ * call: 333 tokens 38.0 -> 25.3 us, 700 tokens 70.0 -> 35.9; 1024 x 4096, 64
+ * tokens 22.8 -> 16.1, 1,300 tokens 61.4 -> 28.0 (k_grouped2 and the seam
+ * GEMM). */
+namespace {
+
+constexpr int D8_KMAX = 64 * KC;
+constexpr int D8_W = 128 * KC;                         /* weight bytes of a stage */
+
+template <int T> struct D8 {
+    static constexpr int WT = T >= 4 ? 2 : 1, NWAVE = 4 * WT;      /* 4 waves along rows, WT along tokens */
+    static constexpr int U = T / WT;                   /* 16-token groups of a wave */
+    static constexpr int STAGE = D8_W + 16 * T * KC * 2;
+    static constexpr int NST = T == 1 ? 4 : T == 2 ? 3 : T == 3 ? 5 : 4;
+    static constexpr int LDS = NST * STAGE;
+    static constexpr int LW = 16 / NWAVE, LX = 4 * T / NWAVE;      /* a wave's loads a stage  */
+    static constexpr int VM = LW + LX;
+    static_assert(LDS <= 160 * 1024 && (NST - 1) * VM < 64 && T % WT == 0, "ring");
+};
+
+template <int N>
+__device__ __forceinline__ void d8_wait()
+{
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+
+} // namespace
+
+template <bool SWIGLU, bool WF32S, int T>
+__global__ __launch_bounds__(64 * D8<T>::NWAVE) void k_dense8(GroupedArgs a)
+{
+    using C = D8<T>;
+    constexpr int FEAT = SWIGLU ? 64 : 128;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int lane = threadIdx.x & 63, wave = wave_in_group();
+    const int rr = lane & 15, gq = lane >> 4, wr = wave & 3, wt = wave >> 2;
+    constexpr int U = C::U;
+    const int K = a.K, N = a.N, M = a.nrows;
+    const int mt = (M + 16 * T - 1) / (16 * T), nslab = N / FEAT, nst = K / KC;
+    /* the slabs of one XCD (workgroups go round the eight) side by side, each
+     * with all its token tiles: W is then fetched into one L2 only */
+    int lin = blockIdx.x;
+    if (nslab % 8 == 0) lin = (lin % 8) * (nslab / 8 * mt) + lin / 8;
+    const int f0 = lin / mt * FEAT, m0 = lin % mt * (16 * T);
+
+    const bool w_up = SWIGLU && wave >= C::NWAVE / 2;             /* staged rows 64 .. 127 are w3's */
+    const __amdgpu_buffer_rsrc_t rw = buf_rsrc(w_up ? a.m3.w : a.m1.w, (uint32_t)N * (uint32_t)K);
+    const __amdgpu_buffer_rsrc_t rx = buf_rsrc(a.B, (uint32_t)M * (uint32_t)K * 2u);
+    uint32_t wo[C::LW], xo[C::LX];
+#pragma unroll
+    for (int i = 0; i < C::LW; i++) {
+        const int r = 8 * (C::LW * wave + i) + lane / 8;
+        wo[i] = (uint32_t)(f0 + (SWIGLU ? r & 63 : r)) * (uint32_t)K + 16u * (uint32_t)swz_w4(r, lane & 7);
+    }
+#pragma unroll
+    for (int i = 0; i < C::LX; i++) {
+        const int r = 4 * (C::LX * wave + i) + lane / 16;
+        xo[i] = m0 + r < M ? (uint32_t)(m0 + r) * (uint32_t)K * 2u + 16u * (uint32_t)swz_b(r, lane & 15) : OOB_OFFSET;
+    }
+    /* load i of a wave's share of stage st; past the end zeros, no traffic */
+    auto issue = [&](int st, int slot, int i) {
+        const uint32_t oob = st < nst ? 0u : OOB_OFFSET;
+        uint8_t *buf = lds + slot * C::STAGE;
+        if (i < C::LW) bdma16(rw, wo[min(i, C::LW - 1)] | oob, st * KC, buf + 1024 * (C::LW * wave + i));
+        else bdma16(rx, xo[max(i - C::LW, 0)] | oob, st * KC * 2, buf + D8_W + 1024 * (C::LX * wave + i - C::LW));
+    };
+    uint32_t wsc[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const void *s = SWIGLU && i ? a.m3.s : a.m1.s;
+        const size_t si = (size_t)(f0 / 128) * nst + min(lane, nst - 1);
+        wsc[i] = WF32S ? __float_as_uint(ld_f32(s, si)) : __float_as_uint(dev_e8m0(ld_u8(s, si)));
+    }
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(wsc[0]), "+v"(wsc[1]));     /* their wait before the ring's loads */
+#endif
+#pragma unroll
+    for (int s = 0; s < C::NST; s++)
+#pragma unroll
+        for (int i = 0; i < C::VM; i++) issue(s, s, i);
+
+    /* this wave's operands of a stage */
+    struct Op { u32x4 w[2][2]; h8 x[4][U]; };
+    const int wrow[2] = {SWIGLU ? 16 * wr + rr : 32 * wr + rr, SWIGLU ? 64 + 16 * wr + rr : 32 * wr + 16 + rr};
+    auto read_w = [&](Op &o, const uint8_t *buf, int h, int i) {
+        o.w[h][i] = *(const u32x4 *)(buf + wrow[i] * KC + 16 * swz_w4(wrow[i], 4 * h + gq));
+    };
+    auto read_x = [&](Op &o, const uint8_t *buf, int j, int u) {
+        const int t = 16 * (U * wt + u) + rr;
+        o.x[j][u] = *(const h8 *)(buf + D8_W + t * (2 * KC) + 16 * swz_b(t, 8 * (j >> 1) + 2 * gq + (j & 1)));
+    };
+    auto decode = [&](h8 (&av)[2], const Op &o, int j) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const u32x4 wv[2] = {o.w[j >> 1][i], o.w[j >> 1][i]};
+            av[i] = a_operand<FMT_FP8_E8M0>(wv, 1.0f, j & 1);
+        }
+    };
+    f4v acc[2][U], part[2][U];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int u = 0; u < U; u++) acc[i][u] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+    int slot = 0;                                      /* of the stage multiplied next */
+    auto step = [&](const Op &cur, Op &nxt, int st) {
+        /* this stage's operands are in registers, and this wave's loads of
+         * the next stage have landed; after the barrier every wave's */
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        d8_wait<(C::NST - 2) * C::VM>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int free = slot;
+        slot = slot + 1 == C::NST ? 0 : slot + 1;
+        const uint8_t *buf = lds + slot * C::STAGE;
+        h8 av[2][2];                                   /* decoded a step ahead */
+        decode(av[0], cur, 0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int i = 0; i < C::VM; i++)
+                    if (1 + i * (4 * U - 1) / C::VM == U * j + u) issue(st + C::NST, free, i);
+                read_x(nxt, buf, j, u);
+                if ((j & 1) == 0 && u == 0) read_w(nxt, buf, j >> 1, 0);
+                if ((j & 1) == 0 && u == U - 1) read_w(nxt, buf, j >> 1, 1);
+                part[0][u] = mfma16(av[j & 1][0], cur.x[j][u], j == 0 ? f4v{0.0f, 0.0f, 0.0f, 0.0f} : part[0][u]);
+                if (u == 0 && j < 3) decode(av[(j + 1) & 1], cur, j + 1);
+                part[1][u] = mfma16(av[j & 1][1], cur.x[j][u], j == 0 ? f4v{0.0f, 0.0f, 0.0f, 0.0f} : part[1][u]);
+                DSV4_ORDER();
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const float sw = st < nst ? __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)wsc[i], st)) : 0.0f;
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[i][u][e] = fmaf(part[i][u][e], sw, acc[i][u][e]);
+        }
+        DSV4_ORDER();
+    };
+
+    d8_wait<(C::NST - 1) * C::VM>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    Op o0, o1;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (j < 2) { read_w(o0, lds, j, 0); read_w(o0, lds, j, 1); }
+#pragma unroll
+        for (int u = 0; u < U; u++) read_x(o0, lds, j, u);
+    }
+    for (int st = 0; st < nst; st += 2) {
+        step(o0, o1, st);
+        step(o1, o0, st + 1);
+    }
+    d8_wait<0>();                                      /* the loads past the end */
+
+    unsigned range_bad = 0;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int m = m0 + 16 * (U * wt + u) + rr;
+        if (m >= M) continue;
+        const int ex = a.bexp ? a.bexp[m] : 0;
+        if constexpr (SWIGLU) {
+            *(uint2 *)((uint16_t *)a.out + (size_t)m * N + f0 + 16 * wr + 4 * gq) =
+                swiglu_f16x4(acc[0][u], acc[1][u], ex, a.limit, range_bad);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                *(f4v *)((float *)a.out + (size_t)m * N + f0 + 32 * wr + 16 * i + 4 * gq) = unscale4(acc[i][u], ex);
+        }
+    }
+    if (range_bad) atomicOr(a.status, range_bad);
+}
+
 /* ------------------------------------------------------------- combine --- */
 
 /* 4 consecutive outputs of one token per thread. The positions and weights
@@ -1597,6 +1790,73 @@ static hipError_t grouped2(const GroupedArgs &a, long items, hipStream_t st)
     return grouped2_ns<WF, SW, TT, g2_stages<WF, TT>()>(a, items, st);
 }
 
+template <bool SW, bool WS, int T>
+static hipError_t dense8_t(const GroupedArgs &a, hipStream_t st)
+{
+    static bool attr_done = false;
+    if (!attr_done) {
+        const hipError_t e = hipFuncSetAttribute((const void *)k_dense8<SW, WS, T>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, D8<T>::LDS);
+        if (e != hipSuccess) return e;
+        attr_done = true;
+    }
+    const long items = (long)((a.nrows + 16 * T - 1) / (16 * T)) * (a.N / (SW ? 64 : 128));
+    constexpr int lds_bytes = D8<T>::LDS;
+    hipLaunchKernelGGL((k_dense8<SW, WS, T>), dim3((unsigned)items), dim3(64 * D8<T>::NWAVE), lds_bytes, st, a);
+    return hipGetLastError();
+}
+
+/* The 16-token groups T of a k_dense8 tile with the least cost: a round of 256
+ * workgroups takes 8, 11, 16, 19 or 26 us with T = 1, 2, 3, 4 or 6 for 4,096
+ * columns (tiles smaller than their share re-read the weights, larger ones
+ * leave CUs idle). 4096 x 4096, us of the call with T = 1 / 2 / 3 / 4 / 6: 77
+ * tokens 16.5 / 19.9 / 21.9 / 23.6 / 27.3, 333 tokens 33.4 / 28.6 / 25.3 / 26.6
+ * / 30.6, 700 tokens 56.6 / 44.4 / 45.3 / 48.1 / 35.9. */
+static int dense8_tile(int M, long slabs, long *cost)
+{
+    const int t[5] = {1, 2, 3, 4, 6}, c[5] = {8, 11, 16, 19, 26};
+    int best = 0;
+    for (int i = 0; i < 5; i++) {
+        const long v = c[i] * ((((long)M + 16 * t[i] - 1) / (16 * t[i]) * slabs + 255) / 256);
+        if (!best || v < *cost) {
+            best = t[i];
+            *cost = v;
+        }
+    }
+    return best;
+}
+
+/* k_dense8 takes rows of up to its scale register's 64 blocks, weights on
+ * 16-byte boundaries and 31-bit offsets; what its callers' other forms flag
+ * in the kernel goes to those. */
+long grouped_dense_cost(const GroupedArgs &a, int fmt, bool swiglu)
+{
+    auto ok = [&](const DSV4QMat &m) {
+        return m.rows == a.N && m.cols == a.K && m.w && m.s && ((uintptr_t)m.w & 15) == 0 && m.blk_r == 128 &&
+               m.blk_c == 128 && m.wdt == (fmt == FMT_FP8_F32S ? DSV4_WFP8_F32S : DSV4_WFP8);
+    };
+    if (a.table || (fmt != FMT_FP8_E8M0 && fmt != FMT_FP8_F32S) || a.K % KC || a.K > D8_KMAX || a.N % 128 ||
+        a.nrows <= 0 || !ok(a.m1) || (swiglu && !ok(a.m3)) || (size_t)a.nrows * a.K * 2 >= (1u << 31) ||
+        (size_t)a.N * a.K >= (1u << 31))
+        return 0;
+    long cost = 0;
+    dense8_tile(a.nrows, a.N / (swiglu ? 64 : 128), &cost);
+    return cost;
+}
+
+template <bool WS, bool SW>
+static hipError_t dense8(const GroupedArgs &a, hipStream_t st)
+{
+    long cost;
+    switch (dense8_tile(a.nrows, a.N / (SW ? 64 : 128), &cost)) {
+    case 1: return dense8_t<SW, WS, 1>(a, st);
+    case 2: return dense8_t<SW, WS, 2>(a, st);
+    case 3: return dense8_t<SW, WS, 3>(a, st);
+    case 4: return dense8_t<SW, WS, 4>(a, st);
+    default: return dense8_t<SW, WS, 6>(a, st);
+    }
+}
+
 template <int WF, bool SW>
 static hipError_t grouped_tt(const GroupedArgs &a, int tt, long items, hipStream_t st)
 {
@@ -1651,6 +1911,11 @@ hipError_t grouped_launch(int fmt, bool swiglu, int tt, const GroupedArgs &a, lo
             return hipErrorInvalidValue;
         const long items = max_tiles * (a.N / (swiglu ? 64 : 128));
         return swiglu ? grouped_w<true>(a, items, st) : grouped_w<false>(a, items, st);
+    }
+    if (tt == GROUPED_DENSE) {
+        if (!grouped_dense_cost(a, fmt, swiglu)) return hipErrorInvalidValue;
+        if (fmt == FMT_FP8_F32S) return swiglu ? dense8<true, true>(a, st) : dense8<true, false>(a, st);
+        return swiglu ? dense8<false, true>(a, st) : dense8<false, false>(a, st);
     }
     if (tt == 8) {
         /* 128-token tiles: FP4 only; byte offsets of every buffer fit 31 bits */

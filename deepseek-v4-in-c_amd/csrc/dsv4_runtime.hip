@@ -686,16 +686,16 @@ void *dsv4_hip_device_ptr(const void *p)
  * every nt. From MMQ_MFMA_MIN_TOKENS tokens on, packed matrices the grouped
  * kernel takes (rows, cols multiples of 128; FP8 with 128x128 blocks or FP4
  * with 1x32) run as one dense fp16-MFMA GEMM (x row-scaled by a power of two
- * and rounded to fp16, weights decoded exactly, fp32 accumulation): FP8 in
- * tiles of 64 rows x 16 or 32 tokens while those are few enough
- * (gemm_thin_seam_nt), from MMQ_SEAM_GEMM_MIN_TOKENS tokens on in the
- * GEMM-shaped seam kernel (128 x 256 tiles), else in the grouped kernel with
- * one group (the same bits in all three); fewer tokens run the block-scaled
- * MFMA GEMV where its geometry fits, else the per-token VALU GEMV. The seam
- * kernel's tiles fill the device only from about 2048 tokens (4096 x 4096
- * FP8: 64 us from 128 to 1024 tokens, 79 us at 2048), the grouped form's
- * 64-token tiles from far fewer (59 us at 1024, 82 us at 1536): the switch
- * sits between. */
+ * and rounded to fp16, weights decoded exactly, fp32 accumulation), FP8 by
+ * cost in the dense tiles (k_dense8) or the GEMM-shaped seam kernel (128 x 256
+ * tiles, about 60 us a round of 256 at 4,096 columns: 4096 x 4096, 1,500
+ * tokens 68.1 against 67.2 us dense, 2,048 tokens 77.5 / 108.8; 1024 x 4096,
+ * 2,048 tokens 65.5 / 37.6), FP4 and rows the dense tiles do not take in the
+ * grouped kernel with one group (the same bits in all three; the seam kernel
+ * from MMQ_SEAM_GEMM_MIN_TOKENS there, 4096 x 4096: 64 us from 128 to 1,024
+ * tokens, 79 at 2,048, the grouped form 59 at 1,024, 82 at 1,536); fewer
+ * tokens run the block-scaled MFMA GEMV where its geometry fits, else the
+ * per-token VALU GEMV. */
 constexpr int MMQ_MFMA_MIN_TOKENS = 32;
 constexpr int MMQ_SEAM_GEMM_MIN_TOKENS = 1280;
 /* From this many tokens the block-scaled MFMA GEMV splits x once into its
@@ -730,14 +730,13 @@ static int enqueue_mmq(const DSV4QMat &d, int fmt, const float *x, float *y, int
         uint16_t *x16 = (uint16_t *)g.x16.p;
         int *ex = (int *)((uint8_t *)g.x16.p + xb);
         HIPCHK(to_f16_rows_launch(x16, ex, x, nt, d.cols, st), "x fp16 launch");
-        if (const int tn = fmt != FMT_FP4_E8M0 && aligned16(d.w) ? gemm_thin_seam_nt(nt, d.rows, d.cols) : 0) {
-            SeamGemmArgs sg;
-            sg.X = x16; sg.ex = ex; sg.W = (const uint8_t *)d.w; sg.Sw = d.s; sg.C = y;
-            sg.M = nt; sg.N = d.rows; sg.K = d.cols;
-            HIPCHK(gemm_thin_seam_launch(sg, fmt == FMT_FP8_F32S, tn, st), "seam GEMM launch");
-            return 0;
-        }
-        if (fmt != FMT_FP4_E8M0 && nt >= MMQ_SEAM_GEMM_MIN_TOKENS && aligned16(d.w) &&
+        GroupedArgs a;
+        memset(&a, 0, sizeof a);
+        a.m1 = d; a.nrows = nt; a.B = x16; a.bexp = ex; a.K = d.cols; a.N = d.rows; a.out = y;
+        a.status = g.st;
+        const long dense = grouped_dense_cost(a, fmt, false);
+        const long seam = GROUPED_DENSE_SEAM * (((nt + 127L) / 128 * ((d.rows + 255) / 256) + 255) / 256);
+        if (fmt != FMT_FP4_E8M0 && (dense ? seam < dense : nt >= MMQ_SEAM_GEMM_MIN_TOKENS) && aligned16(d.w) &&
             gemm_seam_ok(nt, d.rows, d.cols)) {
             SeamGemmArgs sg;
             sg.X = x16; sg.ex = ex; sg.W = (const uint8_t *)d.w; sg.Sw = d.s; sg.C = y;
@@ -745,10 +744,10 @@ static int enqueue_mmq(const DSV4QMat &d, int fmt, const float *x, float *y, int
             HIPCHK(gemm_seam_launch(sg, fmt == FMT_FP8_F32S, st), "seam GEMM launch");
             return 0;
         }
-        GroupedArgs a;
-        memset(&a, 0, sizeof a);
-        a.m1 = d; a.nrows = nt; a.B = x16; a.bexp = ex; a.K = d.cols; a.N = d.rows; a.out = y;
-        a.status = g.st;
+        if (dense) {
+            HIPCHK(grouped_launch(fmt, false, GROUPED_DENSE, a, 1, st), "dense MFMA launch");
+            return 0;
+        }
         /* 16-token tiles give a small batch more workgroups (4096 x 4096
          * FP8: 23 us from 32 to 128 tokens, against 28-32 us in 64-token
          * tiles), 64-token tiles reuse each weight chunk more from about 200
@@ -1500,6 +1499,19 @@ static int grouped_tt(long pairs, int n_experts, int n, int hidden, int inter)
     return pairs <= 16L * n_experts ? 1 : 8;
 }
 
+/* A shared expert's matrix beside the routed ones: an FP8 one over many tokens
+ * in the dense tiles (701 tokens, the call: 890 -> 846 us, 2,048: 1,546 ->
+ * 1,454; up to 192 the 16- and 64-row tiles disturb the routed launches less:
+ * 150 tokens 446 against 451 us). */
+static int enqueue_dense(int fmt, bool swiglu, const GroupedArgs &a, hipStream_t st, const char *what)
+{
+    int tt = a.nrows <= 64 ? 1 : 4;          /* enough workgroups for a small batch */
+    if (a.nrows > 192 && grouped_dense_cost(a, fmt, swiglu)) tt = GROUPED_DENSE;
+    const long rows = tt == GROUPED_DENSE ? a.nrows : grouped_rows_per_tile(tt);
+    HIPCHK(grouped_launch(fmt, swiglu, tt, a, (a.nrows + rows - 1) / rows, st), what);
+    return 0;
+}
+
 static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4ExpertW *table,
                         int n_experts, const int *idx, const float *w, int topk,
                         const DSV4ExpertW *shared, int sfmt, int sinter, int hidden,
@@ -1565,15 +1577,13 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     if (shared) {
         uint16_t *smid = (uint16_t *)(ws + o_smid);
         ys = (float *)(ws + o_ys);
-        const int stt = n <= 64 ? 1 : 4;     /* enough workgroups for a small batch */
-        const long stiles = (n + grouped_rows_per_tile(stt) - 1) / grouped_rows_per_tile(stt);
         GroupedArgs sa;
         memset(&sa, 0, sizeof sa);
         sa.m1 = shared->w1; sa.m3 = shared->w3; sa.nrows = n; sa.B = x16; sa.bexp = ex;
         sa.K = hidden; sa.N = sinter; sa.out = smid; sa.limit = limit; sa.status = g.st;
-        HIPCHK(grouped_launch(sfmt, true, stt, sa, stiles, g.side), "shared gate/up launch");
+        if (enqueue_dense(sfmt, true, sa, g.side, "shared gate/up launch")) return -1;
         sa.m1 = shared->w2; sa.B = smid; sa.bexp = nullptr; sa.K = sinter; sa.N = hidden; sa.out = ys;
-        HIPCHK(grouped_launch(sfmt, false, stt, sa, stiles, g.side), "shared down launch");
+        if (enqueue_dense(sfmt, false, sa, g.side, "shared down launch")) return -1;
         HIPCHK(hipEventRecord(g.join, g.side), "join record");
     }
 

@@ -361,27 +361,28 @@ def test_seam_gemm_bits_equal_grouped_form(lib, pkg, oracle, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["fp8", "fp8f"])
-@pytest.mark.parametrize("rows,cols", [(2048, 128), (2176, 640), (2048, 1152)])
-def test_seam_tile_sizes_same_bits(lib, pkg, oracle, rows, cols, fmt):
-    """The three forms of the FP8 seam give a token the same bits: 16- and
-    32-token tiles of 64 features (both edges of each, a part of a group of
-    reduction blocks, feature tiles no multiple of eight), the grouped form
-    above them and the 128 x 256 tiles from 1280 tokens."""
+@pytest.mark.parametrize("rows,cols,tokens", [
+    (2048, 128, (32, 33, 129, 257, 300, 513, 600, 1000, 1290, 4096)),     # every tile height, then 128 x 256
+    (2176, 640, (32, 47, 300, 500, 700, 1290)),                            # rows no multiple of eight tiles
+    (1024, 8192, (33, 600)),                                               # the longest rows of the dense tiles
+    (128, 8448, (40, 300, 1290)),                                          # past them: grouped form, 128 x 256
+])
+def test_seam_tile_sizes_same_bits(lib, pkg, oracle, rows, cols, tokens, fmt):
+    """The forms of the FP8 seam give a token the same bits: the dense tiles of
+    16 to 96 tokens, the grouped form and the 128 x 256 tiles."""
     rng = np.random.default_rng(rows + cols + len(fmt))
     m, want_of = _fp8_resident(lib, pkg, oracle, fmt, rng, rows, cols)
-    nt = 1290
-    x = rng.standard_normal((nt, cols)).astype(np.float32)
+    x = rng.standard_normal((tokens[-1], cols)).astype(np.float32)
     x[0] *= 1e5
     x[1] *= 1e-9
     x[2] = 0.0
     x = np.ascontiguousarray(x)
-    got = {n: lib.mmq_n(m.desc, np.ascontiguousarray(x[:n].reshape(-1)), n).reshape(n, rows)
-           for n in (32, 33, 128, 129, 147, 300, 400, 1279, nt)}
-    want = want_of(np.ascontiguousarray(x[:33].reshape(-1)), 33).reshape(33, rows)
-    for t in range(33):
-        assert rel_l2(got[33][t], want[t]) <= REL_L2_TOL, t
+    got = {n: lib.mmq_n(m.desc, np.ascontiguousarray(x[:n].reshape(-1)), n).reshape(n, rows) for n in tokens}
+    want = want_of(np.ascontiguousarray(x[:17].reshape(-1)), 17).reshape(17, rows)
+    for t in range(17):
+        assert rel_l2(got[tokens[0]][t], want[t]) <= REL_L2_TOL, t
     for n, y in got.items():
-        assert np.array_equal(bits(y), bits(got[nt][:n])), n
+        assert np.array_equal(bits(y), bits(got[tokens[-1]][:n])), n
     m.drop()
 
 

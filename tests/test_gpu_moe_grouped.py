@@ -534,3 +534,24 @@ def test_grouped_dword_aligned_experts(lib, pkg, oracle, counts, hidden, inter):
     want = oracle_tokens(oracle, experts, None, x, idx, w, list(range(len(x))))
     e = rel_l2(got, want)
     assert e <= REL_L2_TOL, f"rel L2 {e:.3e} (max abs {max_abs(got, want):.3e})"
+
+
+@pytest.mark.parametrize("fmt", ["fp8f32", "fp8e8m0"])
+@pytest.mark.parametrize("hidden,inter,tokens", [(256, 2048, (64, 150, 193, 333, 450, 700)), (512, 640, (40, 210))])
+def test_shared_tile_sizes_same_bits(lib, pkg, oracle, hidden, inter, tokens, fmt):
+    """An FP8 shared expert gives a token the same bits from the 16- and 64-row
+    tiles as from the dense tiles of 16 to 96 tokens above 192 tokens (the
+    routed expert's weight is zero, so the output is the shared one's)."""
+    dgen = torch.Generator(device=DEV).manual_seed(hidden + inter)
+    experts = [DevExpert(lib, pkg, "fp4", inter, hidden, dgen)]
+    shared = DevExpert(lib, pkg, fmt, inter, hidden, dgen)
+    x = bf16_rows(torch.Generator().manual_seed(hidden), tokens[-1], hidden)
+    got = {}
+    for n in tokens:
+        idx, w = np.zeros((n, 1), np.int32), np.zeros((n, 1), np.float32)
+        got[n] = run_dev(lib, experts, shared, x[:n], idx, w, hidden, inter)
+    want = oracle_tokens(oracle, experts, shared, x, idx, w, list(range(17)))
+    e = rel_l2(got[tokens[0]][:17], want)
+    assert e <= REL_L2_TOL, f"rel L2 {e:.3e}"
+    for n, y in got.items():
+        assert np.array_equal(bits(y), bits(got[tokens[-1]][:n])), n
