@@ -304,6 +304,38 @@ def test_mmq_n_presplit_shapes(lib, pkg, oracle, fmt, rows, cols, nt):
     m.drop()
 
 
+@pytest.mark.parametrize("fmt,rows,cols,nt", [
+    ("bf16", 5, 128, 1),             # 20 bytes out: no multiple of 16
+    ("bf16", 1, 8, 3),
+    ("fp8", 128, 4096, 256),         # x fills the host calls' staging exactly
+    ("fp8", 128, 4096, 257),         # and no longer fits
+    ("fp8", 4096, 128, 257),         # y no longer fits
+])
+def test_host_call_staging(lib, pkg, oracle, fmt, rows, cols, nt):
+    """A host-pointer call's bits are the device-pointer call's, whatever part
+    of its operands goes through the pinned staging."""
+    rng = np.random.default_rng(rows + cols + nt)
+    x = rng.standard_normal(nt * cols).astype(np.float32)
+    if fmt == "bf16":
+        W = (rng.standard_normal(rows * cols).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        m = ResidentBf16(lib, pkg, W, rows, cols)
+        dS = None
+    else:
+        W, S = oracle.quant_fp8_blk128((rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+        m = Resident(lib, pkg, pkg.DSV4_WFP8_F32S, W, S, rows, cols, 128, 128)
+        dS = torch.from_numpy(np.ascontiguousarray(S)).cuda()
+    dW = torch.from_numpy(np.ascontiguousarray(W).view(np.uint8)).cuda()
+    dx, dy = torch.from_numpy(x).cuda(), torch.empty(nt * rows, device="cuda")
+    d = pkg.qmat(m.desc.wdt, dW.data_ptr(), dS.data_ptr() if dS is not None else None, rows, cols, m.desc.blk_r,
+                 m.desc.blk_c)
+    lib.mmq_n_dev(dy.data_ptr(), dx.data_ptr(), d, nt)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        got = lib.mmq_n(m.desc, x, nt)
+        assert np.array_equal(bits(got).reshape(-1), bits(dy.cpu().numpy()))
+    m.drop()
+
+
 # ------------------------------------------------------ seam GEMM (FP8) ----
 
 def _fp8_resident(lib, pkg, oracle, fmt, rng, rows, cols):
