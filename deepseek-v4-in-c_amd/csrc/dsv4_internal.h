@@ -395,9 +395,17 @@ inline size_t route_chist_bytes(long npairs, int n_experts)
 {
     return (size_t)((npairs + 1023) / 1024) * (size_t)n_experts * 4;
 }
-hipError_t moe_route_launch(const RouteArgs &a, hipStream_t st);
+/* x16 (rows > 0): the launch's first kernel also converts the rows of x to
+ * scaled fp16 (as to_f16_rows_launch), in workgroups of its own */
+struct RowsF16Args {
+    uint16_t *o;
+    int *ex;
+    const float *x;
+    int rows, cols;
+};
+hipError_t moe_route_launch(const RouteArgs &a, const RowsF16Args &x16, hipStream_t st);
 
-/* dsv4_route for n tokens, one wavefront each: scores [n][scores_ld] fp32
+/* dsv4_route for n tokens, one workgroup each: scores [n][scores_ld] fp32
  * (the gate matvec's output) -> idx, w [n][topk], orig [n][n_experts] (may
  * be NULL). bias [n_experts] may be NULL. With tid2eid ([n_vocab][topk]
  * int64) the ids are tid2eid[token], token = token_ids[t] (device) or

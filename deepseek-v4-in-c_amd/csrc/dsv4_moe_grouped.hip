@@ -168,6 +168,56 @@ __device__ __forceinline__ bool qmat_matches(const DSV4QMat &m, int rows, int co
 
 } // namespace
 
+/* ----------------------------------------------------- rows to fp16 --- */
+
+/* One workgroup of NTHR threads converts a row: the row's largest finite
+ * magnitude (a fixed-order max, order does not matter), then 8 floats -> 8
+ * fp16 per thread and unit, each multiplied by the row's power of two first
+ * (exact). The second pass re-reads the row from cache. */
+__device__ __forceinline__ float finite_abs(float v)
+{
+    const float m = __builtin_fabsf(v);
+    return __builtin_isfinite(m) ? m : 0.0f;
+}
+
+template <int NTHR>
+__device__ __forceinline__ void row_to_f16(uint16_t *o, int *ex, const float *x, int row, int cols, float *wmax)
+{
+    const float *xr = x + (size_t)row * cols;
+    uint16_t *orow = o + (size_t)row * cols;
+    const int units = cols / 8;
+    float m = 0.0f;
+    for (int u = threadIdx.x; u < units; u += NTHR) {
+        const f32x4 a = *(const f32x4 *)(xr + 8 * u), b = *(const f32x4 *)(xr + 8 * u + 4);
+        m = fmaxf(m, fmaxf(fmaxf(finite_abs(a.x), finite_abs(a.y)), fmaxf(finite_abs(a.z), finite_abs(a.w))));
+        m = fmaxf(m, fmaxf(fmaxf(finite_abs(b.x), finite_abs(b.y)), fmaxf(finite_abs(b.z), finite_abs(b.w))));
+    }
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) m = fmaxf(m, __shfl_xor(m, s, 64));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = wmax[0];
+#pragma unroll
+    for (int w = 1; w < NTHR / 64; w++) m = fmaxf(m, wmax[w]);
+    const int e = m > 0.0f ? 14 - ilogbf(m) : 0;       /* m * 2^e in [2^14, 2^15) */
+    if (threadIdx.x == 0) ex[row] = e;
+    for (int u = threadIdx.x; u < units; u += NTHR) {
+        const f32x4 a = *(const f32x4 *)(xr + 8 * u), b = *(const f32x4 *)(xr + 8 * u + 4);
+        u32x4 v;
+        v.x = f16_bits(ldexpf(a.x, e)) | (f16_bits(ldexpf(a.y, e)) << 16);
+        v.y = f16_bits(ldexpf(a.z, e)) | (f16_bits(ldexpf(a.w, e)) << 16);
+        v.z = f16_bits(ldexpf(b.x, e)) | (f16_bits(ldexpf(b.y, e)) << 16);
+        v.w = f16_bits(ldexpf(b.z, e)) | (f16_bits(ldexpf(b.w, e)) << 16);
+        *(u32x4 *)(orow + 8 * u) = v;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_to_f16_rows(uint16_t *o, int *ex, const float *x, int cols)
+{
+    __shared__ float wmax[4];
+    row_to_f16<256>(o, ex, x, blockIdx.x, cols, wmax);
+}
+
 /* ------------------------------------------------------------ routing --- */
 
 /* Chunks of 1024 pairs whose routing ids a thread holds in registers at
@@ -214,11 +264,16 @@ __device__ __forceinline__ int route_leader_count(int e, int E, uint64_t below)
 }
 
 /* Pass one of the two-launch form: workgroup c counts chunk c's pairs per
- * expert into chist[c][E] (and reports bad ids). */
-__global__ __launch_bounds__(1024) void k_moe_route_count(RouteArgs a)
+ * expert into chist[c][E] (and reports bad ids). The workgroups from nch on
+ * convert a row of x each. */
+__global__ __launch_bounds__(1024) void k_moe_route_count(RouteArgs a, int nch, RowsF16Args x16)
 {
     __shared__ int hist[MAX_ROUTE_EXPERTS];
     const int tid = threadIdx.x, E = a.n_experts, c = blockIdx.x;
+    if (c >= nch) {
+        row_to_f16<1024>(x16.o, x16.ex, x16.x, c - nch, x16.cols, (float *)hist);
+        return;
+    }
     const int lane = tid & 63;
     const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
     const int p = c * 1024 + tid;
@@ -240,9 +295,10 @@ __global__ __launch_bounds__(1024) void k_moe_route_count(RouteArgs a)
  * launch, no workgroup waits for another: the form for a few chunks).
  * Workgroup 0 also writes grp_off and tile_pre, every workgroup a share
  * of the tile records; bad ids are
- * reported by workgroup 0 (one launch) or by the counting pass. */
+ * reported by workgroup 0 (one launch) or by the counting pass. The
+ * workgroups from nblk on convert a row of x each (one launch). */
 template <bool PRECOUNT>
-__global__ __launch_bounds__(1024) void k_moe_route(RouteArgs a, int cpb)
+__global__ __launch_bounds__(1024) void k_moe_route(RouteArgs a, int cpb, int nblk, RowsF16Args x16)
 {
     __shared__ int hist[MAX_ROUTE_EXPERTS], before[MAX_ROUTE_EXPERTS];
     __shared__ int cur[MAX_ROUTE_EXPERTS];
@@ -250,6 +306,10 @@ __global__ __launch_bounds__(1024) void k_moe_route(RouteArgs a, int cpb)
     __shared__ unsigned short wcnt[16][MAX_ROUTE_EXPERTS];
     const int tid = threadIdx.x;
     const int E = a.n_experts;
+    if (!PRECOUNT && (int)blockIdx.x >= nblk) {
+        row_to_f16<1024>(x16.o, x16.ex, x16.x, blockIdx.x - nblk, x16.cols, (float *)hist);
+        return;
+    }
     const int nch = (a.npairs + 1023) / 1024;
     const int c_lo = blockIdx.x * cpb, c_hi = min(nch, c_lo + cpb);
     int ev[ROUTE_BATCH];
@@ -337,7 +397,7 @@ __global__ __launch_bounds__(1024) void k_moe_route(RouteArgs a, int cpb)
     /* each tile's bucket: the first expert whose inclusive tile prefix
      * exceeds it, tiles spread over every workgroup's threads; with the
      * bucket's first row and the tile's rows */
-    for (int t = blockIdx.x * 1024 + tid; t < scan_t[E - 1]; t += gridDim.x * 1024) {
+    for (int t = blockIdx.x * 1024 + tid; t < scan_t[E - 1]; t += nblk * 1024) {
         int lo = 0, hi = E - 1;
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
@@ -416,46 +476,6 @@ __global__ __launch_bounds__(1024) void k_moe_route(RouteArgs a, int cpb)
         }
     }
     if (!PRECOUNT && bad && blockIdx.x == 0) atomicOr(a.status, bad);
-}
-
-/* One workgroup per row: the row's largest finite magnitude (a fixed-order
- * max, order does not matter), then 8 floats -> 8 fp16 per thread and unit,
- * each multiplied by the row's power of two first (exact). The second pass
- * re-reads the row from cache. */
-__device__ __forceinline__ float finite_abs(float v)
-{
-    const float m = __builtin_fabsf(v);
-    return __builtin_isfinite(m) ? m : 0.0f;
-}
-
-__global__ __launch_bounds__(256) void k_to_f16_rows(uint16_t *o, int *ex, const float *x, int cols)
-{
-    __shared__ float wmax[4];
-    const float *xr = x + (size_t)blockIdx.x * cols;
-    uint16_t *orow = o + (size_t)blockIdx.x * cols;
-    const int units = cols / 8;
-    float m = 0.0f;
-    for (int u = threadIdx.x; u < units; u += 256) {
-        const f32x4 a = *(const f32x4 *)(xr + 8 * u), b = *(const f32x4 *)(xr + 8 * u + 4);
-        m = fmaxf(m, fmaxf(fmaxf(finite_abs(a.x), finite_abs(a.y)), fmaxf(finite_abs(a.z), finite_abs(a.w))));
-        m = fmaxf(m, fmaxf(fmaxf(finite_abs(b.x), finite_abs(b.y)), fmaxf(finite_abs(b.z), finite_abs(b.w))));
-    }
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) m = fmaxf(m, __shfl_xor(m, s, 64));
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-    const int e = m > 0.0f ? 14 - ilogbf(m) : 0;       /* m * 2^e in [2^14, 2^15) */
-    if (threadIdx.x == 0) ex[blockIdx.x] = e;
-    for (int u = threadIdx.x; u < units; u += 256) {
-        const f32x4 a = *(const f32x4 *)(xr + 8 * u), b = *(const f32x4 *)(xr + 8 * u + 4);
-        u32x4 v;
-        v.x = f16_bits(ldexpf(a.x, e)) | (f16_bits(ldexpf(a.y, e)) << 16);
-        v.y = f16_bits(ldexpf(a.z, e)) | (f16_bits(ldexpf(a.w, e)) << 16);
-        v.z = f16_bits(ldexpf(b.x, e)) | (f16_bits(ldexpf(b.y, e)) << 16);
-        v.w = f16_bits(ldexpf(b.z, e)) | (f16_bits(ldexpf(b.w, e)) << 16);
-        *(u32x4 *)(orow + 8 * u) = v;
-    }
 }
 
 /* --------------------------------------------------------- grouped GEMM --- */
@@ -1726,17 +1746,17 @@ __global__ __launch_bounds__(256) void k_moe_combine(CombineArgs a)
 
 /* ------------------------------------------------------------ launchers --- */
 
-hipError_t moe_route_launch(const RouteArgs &a, hipStream_t st)
+hipError_t moe_route_launch(const RouteArgs &a, const RowsF16Args &x16, hipStream_t st)
 {
     if (a.n_experts < 1 || a.n_experts > MAX_ROUTE_EXPERTS) return hipErrorInvalidValue;
     const int nch = (a.npairs + 1023) / 1024;
     const int cpb = nch > ROUTE_MAX_BLOCKS ? (nch + ROUTE_MAX_BLOCKS - 1) / ROUTE_MAX_BLOCKS : 1;
     const int blocks = nch > 0 ? (nch + cpb - 1) / cpb : 1;
     if (a.chist && nch >= ROUTE_PRECOUNT_CHUNKS) {
-        hipLaunchKernelGGL(k_moe_route_count, dim3(nch), dim3(1024), 0, st, a);
-        hipLaunchKernelGGL(k_moe_route<true>, dim3(blocks), dim3(1024), 0, st, a, cpb);
+        hipLaunchKernelGGL(k_moe_route_count, dim3(nch + x16.rows), dim3(1024), 0, st, a, nch, x16);
+        hipLaunchKernelGGL(k_moe_route<true>, dim3(blocks), dim3(1024), 0, st, a, cpb, blocks, x16);
     } else {
-        hipLaunchKernelGGL(k_moe_route<false>, dim3(blocks), dim3(1024), 0, st, a, cpb);
+        hipLaunchKernelGGL(k_moe_route<false>, dim3(blocks + x16.rows), dim3(1024), 0, st, a, cpb, blocks, x16);
     }
     return hipGetLastError();
 }

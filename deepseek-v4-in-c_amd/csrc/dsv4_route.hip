@@ -217,25 +217,44 @@ __device__ __forceinline__ const int64_t *hash_row(const GateRouteArgs &a, int t
     return a.tid2eid + (int64_t)tok * a.topk;
 }
 
-/* dsv4_route for n tokens given their scores: one wavefront per token. */
+/* dsv4_route for n tokens given their scores: a workgroup per token, an expert
+ * per thread (and every 256 beyond), so that the scores, the biases and the
+ * exp tables of a token's experts are one latency each; then the first wave
+ * selects. One wave per token with its experts one after another waited them
+ * out NJ times (256 experts: 7 tokens 11.9 -> 5.4 us, 701 tokens 20.4 -> 9.1). */
 template <int NJ>
 __global__ __launch_bounds__(256) void k_route(GateRouteArgs a)
 {
-    const int t = wave_id();
-    if (t >= a.n) return;
+    __shared__ float so[64 * NJ], sbias[64 * NJ];
+    const int t = blockIdx.x;
     const int lane = threadIdx.x & 63;
     const int ne = a.n_experts;
     const float *sc = a.scores + (size_t)t * a.scores_ld;
+    constexpr int NE = (64 * NJ + 255) / 256;          /* experts of a thread */
+    float v[NE], bv[NE];
+#pragma unroll
+    for (int j = 0; j < NE; j++) {
+        const int e = min((int)threadIdx.x + 256 * j, ne - 1);
+        v[j] = sc[e];
+        bv[j] = a.bias ? a.bias[e] : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < NE; j++) {
+        const int e = threadIdx.x + 256 * j;
+        if (e >= ne) continue;
+        const float o = route_orig(v[j]);
+        so[e] = o;
+        sbias[e] = a.bias ? o + bv[j] : o;
+        if (a.orig) a.orig[(size_t)t * ne + e] = o;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
     float og[NJ], bs[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int e = lane + 64 * j;
-        og[j] = bs[j] = 0.0f;
-        if (e >= ne) continue;
-        const float o = route_orig(sc[e]);
-        og[j] = o;
-        bs[j] = a.bias ? o + a.bias[e] : o;
-        if (a.orig) a.orig[(size_t)t * ne + e] = o;
+        og[j] = e < ne ? so[e] : 0.0f;
+        bs[j] = e < ne ? sbias[e] : 0.0f;
     }
     bool hbad;
     const int64_t *hrow = hash_row(a, a.token_ids ? a.token_ids[t] : a.token_id, &hbad);
@@ -320,7 +339,7 @@ hipError_t launch_route_nj(const GateRouteArgs &a, hipStream_t st)
         hipLaunchKernelGGL(k_gate_route_bf16<NJ>, dim3((unsigned)((a.n_experts + 3) / 4)), dim3(256), 0, st, a);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_route<NJ>, dim3((unsigned)((a.n + 3) / 4)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_route<NJ>, dim3((unsigned)a.n), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

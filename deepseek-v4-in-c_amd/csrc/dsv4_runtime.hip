@@ -1577,7 +1577,7 @@ static int enqueue_dense(int fmt, bool swiglu, const GroupedArgs &a, hipStream_t
 static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4ExpertW *table,
                         int n_experts, const int *idx, const float *w, int topk,
                         const DSV4ExpertW *shared, int sfmt, int sinter, int hidden,
-                        int inter, float limit, hipStream_t st)
+                        int inter, float limit, hipStream_t st, bool forked)
 {
     const long P = (long)n * topk;
     int tt = grouped_tt(P, n_experts, n, hidden, inter);
@@ -1596,10 +1596,15 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     const size_t o_ch = take(route_chist_bytes(P, n_experts));
     const size_t o_x16 = take((size_t)n * hidden * 2), o_mid = take((size_t)P * inter * 2);
     const size_t o_y = take((size_t)P * hidden * 4), o_ex = take((size_t)n * 4);
-    size_t o_smid = 0, o_ys = 0;
+    const bool fork_x = (size_t)n * hidden > ((size_t)1 << 22);
+    size_t o_smid = 0, o_ys = 0, o_sx = o_x16, o_sex = o_ex;   /* the side stream's x */
     if (shared) {
         o_smid = take((size_t)n * sinter * 2);
         o_ys = take((size_t)n * hidden * 4);
+        if (!fork_x) {
+            o_sx = take((size_t)n * hidden * 2);
+            o_sex = take((size_t)n * 4);
+        }
     }
     HIPCHK(g.moe_ws.need(off), "grouped MoE workspace");
     uint8_t *ws = (uint8_t *)g.moe_ws.p;
@@ -1608,7 +1613,8 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     int *pos = (int *)(ws + o_pos), *row = (int *)(ws + o_row);
     uint16_t *x16 = (uint16_t *)(ws + o_x16), *mid = (uint16_t *)(ws + o_mid);
     float *y = (float *)(ws + o_y);
-    int *ex = (int *)(ws + o_ex);
+    int *ex = (int *)(ws + o_ex), *sex = (int *)(ws + o_sex);
+    uint16_t *sx16 = (uint16_t *)(ws + o_sx);
 
     RouteArgs ra;
     ra.idx = idx; ra.npairs = (int)P; ra.topk = topk; ra.n_experts = n_experts;
@@ -1617,22 +1623,23 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     ra.row_k = nullptr;
     ra.chist = (int *)(ws + o_ch);
     ra.status = g.st;
-    /* A large x goes to fp16 on the side stream, beside the routing
-     * permutation on this one (neither reads the other's output), and this
-     * stream waits for it before the routed launches. A small one converts
-     * here first: the conversion then takes less than that cross-stream wait
-     * (about 10 us between kernels). Either way the shared expert, which
-     * needs only x16, runs on the side stream after it, overlaps the routed
-     * launches and is joined before the combine. */
-    const bool fork_x = (size_t)n * hidden > ((size_t)1 << 22);
-    if (!fork_x) HIPCHK(to_f16_rows_launch(x16, ex, x, n, hidden, st), "x fp16 launch");
-    HIPCHK(hipEventRecord(g.fork, st), "fork record");
-    HIPCHK(hipStreamWaitEvent(g.side, g.fork, 0), "fork wait");
-    if (fork_x) {
-        HIPCHK(to_f16_rows_launch(x16, ex, x, n, hidden, g.side), "x fp16 launch");
-        HIPCHK(hipEventRecord(g.xq, g.side), "convert record");
+    /* The side stream starts where the call did (before the router, when that
+     * is part of it) and needs nothing but x: it converts x to fp16, runs the
+     * shared expert and is joined before the combine. A large x is converted
+     * only there, beside the routing permutation, and this stream waits for
+     * it before the routed launches; a small one is converted once more by
+     * workgroups of the permutation's launch, which spares that wait (about
+     * 6 us between two kernels of this stream) and the launch. With the
+     * router's own change: 7 tokens behind the router 135 -> 124 us, 20 tokens
+     * without a shared expert 237 -> 225, 64 tokens, routing known, 297 -> 295. */
+    if (shared || fork_x) {
+        if (!forked) HIPCHK(hipEventRecord(g.fork, st), "fork record");
+        HIPCHK(hipStreamWaitEvent(g.side, g.fork, 0), "fork wait");
+        HIPCHK(to_f16_rows_launch(sx16, sex, x, n, hidden, g.side), "x fp16 launch");
     }
-    HIPCHK(moe_route_launch(ra, st), "route launch");
+    if (fork_x) HIPCHK(hipEventRecord(g.xq, g.side), "convert record");
+    RowsF16Args xa = {x16, ex, x, fork_x ? 0 : n, hidden};
+    HIPCHK(moe_route_launch(ra, xa, st), "route launch");
     if (fork_x) HIPCHK(hipStreamWaitEvent(st, g.xq, 0), "convert wait");
 
     float *ys = nullptr;
@@ -1641,7 +1648,7 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
         ys = (float *)(ws + o_ys);
         GroupedArgs sa;
         memset(&sa, 0, sizeof sa);
-        sa.m1 = shared->w1; sa.m3 = shared->w3; sa.nrows = n; sa.B = x16; sa.bexp = ex;
+        sa.m1 = shared->w1; sa.m3 = shared->w3; sa.nrows = n; sa.B = sx16; sa.bexp = sex;
         sa.K = hidden; sa.N = sinter; sa.out = smid; sa.limit = limit; sa.status = g.st;
         if (enqueue_dense(sfmt, true, sa, g.side, "shared gate/up launch")) return -1;
         sa.m1 = shared->w2; sa.B = smid; sa.bexp = nullptr; sa.K = sinter; sa.N = hidden; sa.out = ys;
@@ -1693,7 +1700,7 @@ static int enqueue_shared_fp8q(float *ys, uint8_t *mq, float *ms, const float *x
 static int enqueue_moe_grouped_mx(float *out, const float *x, int n, const DSV4ExpertW *table,
                            int n_experts, const int *idx, const float *w, int topk,
                            const DSV4ExpertW *shared, int sfmt, int sinter, int hidden, int inter,
-                           float limit, hipStream_t st)
+                           float limit, hipStream_t st, bool forked)
 {
     const long P = (long)n * topk;
     const int trows = grouped_mx_rows_per_tile();
@@ -1739,7 +1746,7 @@ static int enqueue_moe_grouped_mx(float *out, const float *x, int n, const DSV4E
     /* x to MXFP8 on the side stream, beside the routing permutation on this
      * one (neither reads the other's output); the shared expert follows it
      * there */
-    HIPCHK(hipEventRecord(g.fork, st), "fork record");
+    if (!forked) HIPCHK(hipEventRecord(g.fork, st), "fork record");
     HIPCHK(hipStreamWaitEvent(g.side, g.fork, 0), "fork wait");
     HIPCHK(quant_act_mxfp8_launch(x8, xs, x, n, hidden, g.side), "x MXFP8 launch");
     HIPCHK(hipEventRecord(g.xq, g.side), "quant record");
@@ -1751,7 +1758,7 @@ static int enqueue_moe_grouped_mx(float *out, const float *x, int n, const DSV4E
     ra.row_k = nullptr;
     ra.chist = (int *)(ws + o_ch);
     ra.status = g.st;
-    HIPCHK(moe_route_launch(ra, st), "route launch");
+    HIPCHK(moe_route_launch(ra, RowsF16Args{}, st), "route launch");
 
     float *ys = nullptr;
     if (sh_fp8) {
@@ -1851,7 +1858,7 @@ int dsv4_hip_moe_grouped_dev(float *out, const float *x, int n, const DSV4Expert
         return -1;
     if (!aligned16(x) || !aligned16(out)) return fail("moe_grouped_dev: x and out must be 16-byte aligned");
     return enqueue_moe_grouped(out, x, n, experts, n_experts, idx, w, topk, shared, sfmt, sinter,
-                               hidden, inter, limit, (hipStream_t)stream);
+                               hidden, inter, limit, (hipStream_t)stream, false);
 }
 
 int dsv4_hip_moe_layer_n_dev(float *out, const float *x, int n, const DSV4QMat *gate,
@@ -1887,6 +1894,9 @@ int dsv4_hip_moe_layer_n_dev(float *out, const float *x, int n, const DSV4QMat *
     float *scores = (float *)g.route.p;
     int *idx = idx_out ? idx_out : (int *)((uint8_t *)g.route.p + sb);
     float *w = w_out ? w_out : (float *)((uint8_t *)g.route.p + sb + rb);
+    /* the call's side stream needs only x: it starts here, beside the router
+     * (2,000 tokens 1,047 -> 1,028 us, MXFP8 1,500 tokens 220 -> 208) */
+    HIPCHK(hipEventRecord(g.fork, st), "fork record");
     if (enqueue_mmq(*gate, gfmt, x, scores, n, st)) return -1;
     GateRouteArgs a;
     memset(&a, 0, sizeof a);
@@ -1905,9 +1915,9 @@ int dsv4_hip_moe_layer_n_dev(float *out, const float *x, int n, const DSV4QMat *
     a.status = g.st;
     HIPCHK(gate_route_launch(a, st), "route launch");
     return mx ? enqueue_moe_grouped_mx(out, x, n, experts, n_experts, idx, w, topk, shared, sfmt, sinter,
-                                       hidden, inter, limit, st)
+                                       hidden, inter, limit, st, true)
               : enqueue_moe_grouped(out, x, n, experts, n_experts, idx, w, topk, shared, sfmt, sinter,
-                                    hidden, inter, limit, st);
+                                    hidden, inter, limit, st, true);
 }
 
 int dsv4_hip_moe_grouped_mx_dev(float *out, const float *x, int n, const DSV4ExpertW *experts,
@@ -1928,7 +1938,7 @@ int dsv4_hip_moe_grouped_mx_dev(float *out, const float *x, int n, const DSV4Exp
     if (!aligned16(x) || !aligned16(out))
         return fail("moe_grouped_mx_dev: x and out must be 16-byte aligned");
     return enqueue_moe_grouped_mx(out, x, n, experts, n_experts, idx, w, topk, shared, sfmt, sinter,
-                                  hidden, inter, limit, (hipStream_t)stream);
+                                  hidden, inter, limit, (hipStream_t)stream, false);
 }
 
 int dsv4_hip_moe_grouped_mx_mid_dev(uint8_t *mid, uint8_t *mid_s, int *row_tok, int *row_k,
@@ -1967,7 +1977,7 @@ int dsv4_hip_moe_grouped_mx_mid_dev(uint8_t *mid, uint8_t *mid_s, int *row_tok, 
     ra.grp_off = (int *)(ws + o_grp); ra.tile_pre = (int *)(ws + o_tp); ra.tile_rec = (TileRec *)(ws + o_tg);
     ra.pos = (int *)(ws + o_pos); ra.row_tok = row_tok; ra.row_k = row_k; ra.status = g.st;
     ra.chist = (int *)(ws + o_ch);
-    HIPCHK(moe_route_launch(ra, st), "route launch");
+    HIPCHK(moe_route_launch(ra, RowsF16Args{}, st), "route launch");
     HIPCHK(quant_act_mxfp8_launch(ws + o_x8, ws + o_xs, x, n, hidden, st), "x MXFP8 launch");
     GroupedMxArgs ga;
     memset(&ga, 0, sizeof ga);
@@ -2044,7 +2054,7 @@ int dsv4_hip_moe_grouped(float *out, const float *x, int n, const int *topk_idx,
         return -1;
     if (enqueue_moe_grouped((float *)g.y.p, (const float *)g.x.p, n, (const DSV4ExpertW *)tp,
                             n_experts, (const int *)(tp + tb), (const float *)(tp + tb + ib), topk,
-                            shared ? &sdev : nullptr, sfmt, sinter, hidden, inter, limit, g.stream))
+                            shared ? &sdev : nullptr, sfmt, sinter, hidden, inter, limit, g.stream, false))
         return -1;
     return finish_host_call(out, g.y.p, (size_t)n * hidden * 4, "moe_grouped");
 }
@@ -2074,7 +2084,7 @@ int dsv4_hip_moe_route_dev(int *ex_off, int *ex_tok, int *ex_k, int *pos, const 
     ra.tile_rec = (TileRec *)((uint8_t *)g.small.p + o_tg);
     ra.pos = pos; ra.row_tok = ex_tok; ra.row_k = ex_k; ra.status = g.st;
     ra.chist = (int *)((uint8_t *)g.small.p + o_ch);
-    HIPCHK(moe_route_launch(ra, (hipStream_t)stream), "route launch");
+    HIPCHK(moe_route_launch(ra, RowsF16Args{}, (hipStream_t)stream), "route launch");
     return 0;
 }
 
