@@ -48,6 +48,7 @@
  * Bound: HBM (each weight byte is read once per call).
  */
 #include "dsv4_internal.h"
+#include "dsv4_gate_route.h"
 
 #include <algorithm>
 #include <cstring>
@@ -1383,17 +1384,16 @@ __device__ __forceinline__ v4f px8_mma(const Px8Tile<FMT, NP> &t, const uint8_t 
  * and ran at 1.2 TB/s). Waves 0-3 take w1, waves 4-7 w3, each over a quarter
  * of K in NP chunk pairs (hidden = 1024 NP <= 4096). */
 template <int FMT, int NP>
-__global__ __launch_bounds__(512) void k_gateup_px8(GateUpMxArgs a)
+__device__ __forceinline__ void gateup_px8_group(const GateUpMxArgs &a, int blk, uint8_t *lds)
 {
-    extern __shared__ __align__(16) uint8_t lds[];
     constexpr int NC = 8 * NP;                         /* chunks of hidden */
     constexpr int UPL = (NC * 16 + 511) / 512;
     const int lane = threadIdx.x & 63;
     const int wave = wave_in_group();
     const int mat = wave >> 2, kq = wave & 3;
     const int tiles = a.inter / 8;
-    const int slot = blockIdx.x / tiles;
-    const int r0 = (blockIdx.x - slot * tiles) * 8;
+    const int slot = blk / tiles;
+    const int r0 = (blk - slot * tiles) * 8;
     const int c0 = kq * 2 * NP;                        /* the wave's first chunk */
     uint8_t *tab = lds;                                /* NC chunks + zero operand */
     float *red = (float *)(lds + NC * TAB_CHUNK + TAB_ZERO);   /* [2 mats][4 quarters][16] */
@@ -1433,6 +1433,28 @@ __global__ __launch_bounds__(512) void k_gateup_px8(GateUpMxArgs a)
         }
         mid[r0 + rr] = dev_swiglu(gs, us, a.limit);
     }
+}
+
+template <int FMT, int NP>
+__global__ __launch_bounds__(512) void k_gateup_px8(GateUpMxArgs a)
+{
+    extern __shared__ __align__(16) uint8_t lds[];
+    gateup_px8_group<FMT, NP>(a, (int)blockIdx.x, lds);
+}
+
+/* A decode token's gate + router and its shared expert's gate/up, which need
+ * only x, in one launch: the first nroute workgroups (four waves of eight)
+ * are the router's, which has the longer chain of latencies. Behind one
+ * another they took 10.4 and 5.7 us and a launch. At most 256 experts. */
+template <int FMT, int NP>
+__global__ __launch_bounds__(512) void k_gate_route_gateup(GateRouteArgs r, GateUpMxArgs a, int nroute)
+{
+    extern __shared__ __align__(16) uint8_t lds[];
+    if ((int)blockIdx.x < nroute) {
+        if (threadIdx.x < 256) gate_route_group<4>(r, (unsigned)nroute, lds);
+        return;
+    }
+    gateup_px8_group<FMT, NP>(a, (int)blockIdx.x - nroute, lds);
 }
 
 /* One-token FP8 matvec in the same 8-row chunk-pair tiles: one workgroup per
@@ -2082,10 +2104,33 @@ hipError_t gateup_px_k(const GateUpMxArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
+template <int NP>
+constexpr size_t gateup_px8_lds() { return (size_t)8 * NP * TAB_CHUNK + TAB_ZERO + 2 * 4 * 16 * 4; }
+
+template <int FMT, int NP>
+hipError_t gate_route_gateup_k(const GateRouteArgs &r, const GateUpMxArgs &a, hipStream_t st)
+{
+    const size_t lds = std::max<size_t>(gateup_px8_lds<NP>(), b4_lds_bytes(1));
+    const int nroute = (r.n_experts + 3) / 4;
+    hipLaunchKernelGGL((k_gate_route_gateup<FMT, NP>), dim3((unsigned)(nroute + a.inter / 8)), dim3(512), lds, st, r,
+                       a, nroute);
+    return hipGetLastError();
+}
+
+template <int FMT>
+hipError_t gate_route_gateup_fmt(const GateRouteArgs &r, const GateUpMxArgs &a, hipStream_t st)
+{
+    switch (a.hidden) {
+    case 1024: return gate_route_gateup_k<FMT, 1>(r, a, st);
+    case 2048: return gate_route_gateup_k<FMT, 2>(r, a, st);
+    default: return gate_route_gateup_k<FMT, 4>(r, a, st);
+    }
+}
+
 template <int FMT, int NP>
 hipError_t gateup_px8_k(const GateUpMxArgs &a, hipStream_t st)
 {
-    const size_t lds = (size_t)8 * NP * TAB_CHUNK + TAB_ZERO + 2 * 4 * 16 * 4;
+    const size_t lds = gateup_px8_lds<NP>();
     const dim3 grid((unsigned)(a.nslots * (a.inter / 8)));
     hipLaunchKernelGGL((k_gateup_px8<FMT, NP>), grid, dim3(512), lds, st, a);
     return hipGetLastError();
@@ -2249,6 +2294,20 @@ hipError_t gateup_mx_launch(int fmt, GateUpMxArgs a, hipStream_t st)
     case FMT_FP4_E8M0: return gateup_mx_fmt<FMT_FP4_E8M0>(a, st);
     default: return hipErrorInvalidValue;
     }
+}
+
+bool gate_route_gateup_ok(int fmt, const GateRouteArgs &r, const GateUpMxArgs &a)
+{
+    return (fmt == FMT_FP8_E8M0 || fmt == FMT_FP8_F32S) && r.gate_w && r.n_experts <= 256 && gate_route_ok(r) &&
+           a.nslots == 1 && a.use_direct && !a.msplit && a.inter % 128 == 0 &&
+           (a.hidden == 1024 || a.hidden == 2048 || a.hidden == 4096);
+}
+
+hipError_t gate_route_gateup_launch(int fmt, const GateRouteArgs &r, const GateUpMxArgs &a, hipStream_t st)
+{
+    if (!gate_route_gateup_ok(fmt, r, a)) return hipErrorInvalidValue;
+    return fmt == FMT_FP8_F32S ? gate_route_gateup_fmt<FMT_FP8_F32S>(r, a, st)
+                               : gate_route_gateup_fmt<FMT_FP8_E8M0>(r, a, st);
 }
 
 hipError_t down_mx_launch(DownMxArgs a, hipStream_t st)

@@ -441,7 +441,13 @@ struct GateRouteArgs {
     float *ws_orig, *ws_biased, *scores_out;
     unsigned *counter;
 };
+bool gate_route_ok(const GateRouteArgs &a);
 hipError_t gate_route_launch(const GateRouteArgs &a, hipStream_t st);
+/* the fused gate + router (a.gate_w set, at most 256 experts) and an FP8
+ * expert's gate/up of one slot in one launch; hidden 1024, 2048 or 4096 */
+struct GateUpMxArgs;
+bool gate_route_gateup_ok(int fmt, const GateRouteArgs &a, const GateUpMxArgs &u);
+hipError_t gate_route_gateup_launch(int fmt, const GateRouteArgs &a, const GateUpMxArgs &u, hipStream_t st);
 
 /* Row r of x [rows][cols] (cols % 8 == 0, x 16-byte aligned) ->
  * o[r][c] = fp16(x[r][c] * 2^ex[r]) with ex[r] the power of two that puts the

@@ -441,3 +441,44 @@ def test_moe_layer_n_matches_router_and_grouped(lib, pkg, oracle, n, mx, hashed)
         go = got.reshape(n, L.hidden)
         for t in (0, n - 1):
             check_close(go[t], L.want(oracle, xh[t], gi[t], gw[t]), 1e-3)
+
+
+@pytest.mark.parametrize("ne,hidden,inter,topk,hashed", [(256, 4096, 2048, 6, False), (255, 1024, 256, 8, False),
+                                                         (5, 2048, 512, 2, True), (64, 4096, 256, 4, True),
+                                                         (257, 1024, 256, 3, False), (64, 512, 256, 3, False)])
+@pytest.mark.parametrize("fmt", ["fp8f32", "fp8e8m0"])
+def test_moe_layer_router_beside_shared(lib, pkg, ne, hidden, inter, topk, hashed, fmt):
+    """The router in one launch with the FP8 shared expert's gate/up (up to
+    256 experts, hidden 1024 to 4096; beyond, launches of their own): picks
+    and weights are those of a call without a shared expert, the output is
+    moe_decode_dev's for them, bit for bit."""
+    from test_gpu_moe_grouped import DevExpert, table_of
+    dgen = torch.Generator(device=DEV).manual_seed(ne + hidden)
+    few = [DevExpert(lib, pkg, "fp4", inter, hidden, dgen) for _ in range(3)]
+    tbl = table_of([few[e % 3] for e in range(ne)])
+    shared = DevExpert(lib, pkg, fmt, inter, hidden, dgen)
+    gw = (torch.randn(ne, hidden, generator=dgen, device=DEV) * 0.02).bfloat16()
+    gate = pkg.qmat(pkg.DSV4_WBF16, gw.data_ptr(), None, ne, hidden, 0, 0)
+    bias = torch.randn(ne, generator=dgen, device=DEV) * 0.05
+    t2e = torch.from_numpy(np.stack([np.random.default_rng(i).choice(ne, topk, replace=False)
+                                     for i in range(4)]).astype(np.int64)).to(DEV)
+    kw = dict(tid2eid_ptr=t2e.data_ptr(), n_vocab=4, token_id=2) if hashed else dict(bias_ptr=bias.data_ptr())
+    lib.status()
+    for seed in (1, 2):
+        x = dev_f32(bf16_x(seed, hidden))
+        res = []
+        for sh in (None, shared.desc):
+            out = torch.empty(hidden, device=DEV)
+            di = torch.empty(topk, dtype=torch.int32, device=DEV)
+            dw = torch.empty(topk, device=DEV)
+            lib.moe_layer_dev(out.data_ptr(), x.data_ptr(), gate, tbl.data_ptr(), ne, topk, 2.5, sh, hidden, inter,
+                              10.0, idx_ptr=di.data_ptr(), w_ptr=dw.data_ptr(), **kw)
+            torch.cuda.synchronize()
+            res.append((out.cpu().numpy(), di.cpu().numpy(), bits(dw.cpu().numpy())))
+        assert np.array_equal(res[0][1], res[1][1]) and np.array_equal(res[0][2], res[1][2])
+        want = torch.empty(hidden, device=DEV)
+        lib.moe_decode_dev(want.data_ptr(), x.data_ptr(), tbl.data_ptr(), ne, di.data_ptr(), dw.data_ptr(), topk,
+                           shared.desc, hidden, inter, 10.0)
+        torch.cuda.synchronize()
+        assert np.array_equal(bits(res[1][0]), bits(want.cpu().numpy()))
+    assert lib.status() == 0
