@@ -236,6 +236,36 @@ def test_mx_shapes(lib, pkg, oracle, n, topk, ne, zipf, hidden, inter, with_shar
              tokens, smid=smid)
 
 
+@pytest.mark.parametrize("hidden,inter", [(512, 512), (1024, 1536), (4096, 512), (2048, 1024)])
+def test_mx_scale_loads_same_bits(lib, pkg, hidden, inter):
+    """Scales in 16-byte pieces of four stages give the bits of scales a dword
+    at a time, which experts whose scales start 4 bytes past a 16-byte
+    boundary take: buckets around every tile height, one group of stages and
+    more."""
+    counts = [1, 17, 65, 96, 127, 128, 129, 255, 256, 257, 420]
+    dgen = torch.Generator(device=DEV).manual_seed(hidden + inter)
+    experts = [DevExpert(lib, pkg, "fp4", inter, hidden, dgen) for _ in counts]
+    n = sum(counts)
+    idx = np.repeat(np.arange(len(counts), dtype=np.int32), counts).reshape(n, 1)
+    np.random.default_rng(1).shuffle(idx)
+    w = np.ones((n, 1), np.float32)
+    x = bf16_rows(torch.Generator().manual_seed(3), n, hidden)
+    want = run_mx(lib, experts, None, x, idx, w, hidden, inter)[:3]
+    keep = []
+    for e in experts:
+        q = []
+        for m in e.m:
+            S = torch.zeros(m.S.numel() + 32, dtype=torch.uint8, device=DEV)
+            S[4:4 + m.S.numel()] = m.S
+            keep.append(S)
+            d = m.desc
+            q.append(pkg.qmat(d.wdt, m.W.data_ptr(), S.data_ptr() + 4, d.rows, d.cols, d.blk_r, d.blk_c))
+        e.desc = pkg.ExpertW(*q)
+    got = run_mx(lib, experts, None, x, idx, w, hidden, inter)[:3]
+    assert np.all(np.isfinite(want[0])) and np.array_equal(bits(got[0]), bits(want[0]))
+    assert np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2])
+
+
 @pytest.mark.parametrize("limit", [10.0, 0.0])
 def test_mx_swiglu_clamp(lib, pkg, oracle, limit):
     """gate and up of standard deviation 25: the clamp (and its absence)
