@@ -598,7 +598,7 @@ hipError_t gemm_fp8_launch(const GemmArgs &a, bool w_f32s, bool out_bf16, hipStr
     if ((size_t)a.M * a.K > 0xFFFFFFFFull || (size_t)a.N * a.K > 0xFFFFFFFFull ||
         (size_t)a.M * a.sa_tok * 4 + (size_t)(a.K / GK) * a.sa_kb * 4 > 0xFFFFFFFFull)
         return hipErrorInvalidValue;
-    if (const int nt = gemm_thin_nt(a.M, a.N, a.K)) return gemm_thin_fp8_launch(a, w_f32s, out_bf16, nt, st);
+    if (const int t = gemm_mid_tile(a.M, a.N, a.K)) return gemm_mid_fp8_launch(a, w_f32s, out_bf16, t, st);
     if (w_f32s) return out_bf16 ? launch_gemm<true, true>(a, st) : launch_gemm<true, false>(a, st);
     return out_bf16 ? launch_gemm<false, true>(a, st) : launch_gemm<false, false>(a, st);
 }
@@ -610,7 +610,7 @@ hipError_t gemm_mx_launch(const GemmArgs &a, bool out_bf16, hipStream_t st)
         return hipErrorInvalidValue;
     if ((size_t)a.M * a.K > 0xFFFFFFFFull || (size_t)a.N * a.K > 0xFFFFFFFFull)
         return hipErrorInvalidValue;
-    if (const int nt = gemm_thin_nt(a.M, a.N, a.K)) return gemm_thin_mx_launch(a, out_bf16, nt, st);
+    if (const int t = gemm_mid_tile(a.M, a.N, a.K)) return gemm_mid_mx_launch(a, out_bf16, t, st);
     return out_bf16 ? launch_gemm_mx<true>(a, st) : launch_gemm_mx<false>(a, st);
 }
 

@@ -333,12 +333,12 @@ struct SeamGemmArgs {
 bool gemm_seam_ok(int M, int N, int K);
 hipError_t gemm_seam_launch(const SeamGemmArgs &s, bool w_f32s, hipStream_t st);
 
-/* The FP8 and MXFP8 GEMMs in tiles of 64 features x 16 nt tokens
- * (dsv4_gemm_thin.hip); gemm_thin_nt: the nt a shape takes, 0 for the large
+/* The FP8 and MXFP8 GEMMs in tiles of 128 features x 16 t tokens
+ * (dsv4_gemm_mid.hip); gemm_mid_tile: the t a shape takes, 0 for the large
  * tiles. */
-int gemm_thin_nt(int M, int N, int K);
-hipError_t gemm_thin_fp8_launch(const GemmArgs &g, bool w_f32s, bool out_bf16, int nt, hipStream_t st);
-hipError_t gemm_thin_mx_launch(const GemmArgs &g, bool out_bf16, int nt, hipStream_t st);
+int gemm_mid_tile(int M, int N, int K);
+hipError_t gemm_mid_fp8_launch(const GemmArgs &g, bool w_f32s, bool out_bf16, int t, hipStream_t st);
+hipError_t gemm_mid_mx_launch(const GemmArgs &g, bool out_bf16, int t, hipStream_t st);
 
 /* ---------------------------------------------- dequant / quantizers --- */
 hipError_t dequant_launch(int fmt, const DSV4QMat &m, float *out, hipStream_t st);

@@ -195,15 +195,15 @@ def test_gemm_prequantized_matches_fused(lib, pkg, oracle):
     assert np.array_equal(bits(C.cpu().numpy()), bits(fused))
 
 
-@pytest.mark.parametrize("n,k,big", [(1024, 128, 1040), (1024, 1152, 1040), (384, 640, 2740),
-                                     (2048, 8192, 520)])
+@pytest.mark.parametrize("n,k,big", [(1024, 128, 4100), (1024, 1152, 4100), (384, 640, 10890),
+                                     (2048, 8192, 2050)])
 @pytest.mark.parametrize("form", ["fp8f", "fp8", "mx"])
 def test_gemm_tile_sizes_same_bits(lib, pkg, oracle, n, k, big, form):
-    """A token's outputs have the same bits from the 64-feature tiles of 16,
-    32 and 64 tokens (the edges of a tile and of each tile size's range, one
-    block to 64 of the reduction, feature tiles no multiple of eight) as from
-    the 128 x 256 ones, which `big` tokens take; fp32 and bf16 results, and
-    quantized operands as their entry points take them."""
+    """A token's outputs have the same bits from the tiles of 32, 64 and 128
+    tokens (the edges of a tile and of each tile size's range, one block to 64
+    of the reduction, feature tiles no multiple of eight) as from the 128 x 256
+    ones, which `big` tokens take; fp32 and bf16 results, and quantized
+    operands as their entry points take them."""
     rng = np.random.default_rng(n + k + len(form))
     A = rng.standard_normal((big, k)).astype(np.float32)
     W, S = make_weight(oracle, rng, n, k, f32s=form == "fp8f")
@@ -213,10 +213,8 @@ def test_gemm_tile_sizes_same_bits(lib, pkg, oracle, n, k, big, form):
         run = lambda a, ob: run_gemm(lib, pkg, a, W, S, n, k, form == "fp8f", ob, 0)
     want = run(A, 0)
     want_bf16 = run(A, 1)
-    tiles = n // 64
-    edges = {16 * nt * (256 // tiles) for nt in (1, 2, 4)}
-    for m in sorted({1, 15, 16, 17, 33, 65} | edges | {e + 1 for e in edges}):
-        m = min(m, big)
+    edges = {16 * t * (256 // (n // 128)) for t in (2, 4, 8)}
+    for m in sorted({1, 15, 31, 33, 65, 129} | edges | {e + 1 for e in edges if e + 1 < big}):
         assert np.array_equal(bits(run(A[:m], 0)), bits(want[:m])), m
         assert np.array_equal(run(A[:m], 1), want_bf16[:m]), m
     m = 37
