@@ -511,7 +511,9 @@ struct GroupedMxArgs {
     unsigned *status;
 };
 int grouped_mx_rows_per_tile();
-/* fat tiles (more than 64 token rows) on `st`, thin tiles on `st_thin` */
+/* fat tiles (more than 64 token rows) on `st`, thin tiles on `st_thin`; a K
+ * without thin kernel (grouped_mx_has_thin) runs every tile on `st` */
+bool grouped_mx_has_thin(int K);
 hipError_t grouped_mx_launch(bool swiglu, const GroupedMxArgs &a, long max_tiles, hipStream_t st,
                              hipStream_t st_thin);
 

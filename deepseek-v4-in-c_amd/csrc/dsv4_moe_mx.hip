@@ -928,6 +928,9 @@ __global__ __launch_bounds__(256, 2) void k_grouped_mx_thin(GroupedMxArgs a, int
 
 int grouped_mx_rows_per_tile() { return GX_TILE; }
 
+/* the thin ring runs whole groups of stages */
+bool grouped_mx_has_thin(int K) { return K % TH_KQ == 0; }
+
 template <bool SW>
 static hipError_t grouped_mx_k(const GroupedMxArgs &a, long items, int thin_rows, hipStream_t st,
                                hipStream_t st_thin)
@@ -953,7 +956,7 @@ hipError_t grouped_mx_launch(bool swiglu, const GroupedMxArgs &a, long max_tiles
         (size_t)a.N * a.K / 2 >= (1u << 31))
         return hipErrorInvalidValue;
     const long items = max_tiles * (a.N / feat);
-    const int thin_rows = a.K % TH_KQ == 0 ? TH_TOK : 0;   /* the thin ring runs whole groups of stages */
+    const int thin_rows = grouped_mx_has_thin(a.K) ? TH_TOK : 0;
     return swiglu ? grouped_mx_k<true>(a, items, thin_rows, st, st_thin)
                   : grouped_mx_k<false>(a, items, thin_rows, st, st_thin);
 }

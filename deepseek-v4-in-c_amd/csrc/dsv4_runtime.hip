@@ -1804,11 +1804,21 @@ static int enqueue_moe_grouped_mx(float *out, const float *x, int n, const DSV4E
     ga.row_tok = row; ga.B = x8; ga.BS = xs; ga.nrows = n; ga.K = hidden; ga.N = inter;
     ga.out = mid; ga.out_s = ms; ga.limit = limit; ga.status = g.st;
     /* thin tiles (weight streaming) on a second side stream, beside the fat
-     * tiles (MFMA) on this one; each down launch reads only mid rows its own
-     * gate/up launch wrote */
+     * tiles (MFMA) on this one. Each down launch reads only mid rows that its
+     * own stream's gate/up launch wrote, unless one of the two launches has no
+     * thin kernel (its K is no whole number of thin granules): then the down
+     * launch waits for the other stream's gate/up */
     HIPCHK(hipEventRecord(g.fork2, st), "fork record");
     HIPCHK(hipStreamWaitEvent(g.side2, g.fork2, 0), "fork wait");
     HIPCHK(grouped_mx_launch(true, ga, max_tiles, st, g.side2), "routed gate/up launch");
+    const bool thin_up = grouped_mx_has_thin(hidden), thin_down = grouped_mx_has_thin(inter);
+    if (thin_up && !thin_down) {
+        HIPCHK(hipEventRecord(g.join2, g.side2), "mid record");
+        HIPCHK(hipStreamWaitEvent(st, g.join2, 0), "mid wait");
+    } else if (!thin_up && thin_down) {
+        HIPCHK(hipEventRecord(g.fork2, st), "mid record");
+        HIPCHK(hipStreamWaitEvent(g.side2, g.fork2, 0), "mid wait");
+    }
     ga.row_tok = nullptr; ga.B = mid; ga.BS = ms; ga.nrows = (int)P; ga.K = inter; ga.N = hidden;
     ga.out = y; ga.out_s = nullptr;
     HIPCHK(grouped_mx_launch(false, ga, max_tiles, st, g.side2), "routed down launch");

@@ -266,6 +266,29 @@ def test_mx_scale_loads_same_bits(lib, pkg, hidden, inter):
     assert np.array_equal(got[1], want[1]) and np.array_equal(got[2], want[2])
 
 
+@pytest.mark.parametrize("hidden,inter", [(4096, 512), (512, 4096), (1024, 1024)])
+def test_mx_mid_is_this_calls(lib, pkg, hidden, inter):
+    """The down launch waits for the gate/up of every tile, also where only one
+    of the two has thin tiles on a stream of their own: a call on new tokens
+    gives the bits it gives when its workspace already holds their mid."""
+    dgen = torch.Generator(device=DEV).manual_seed(hidden)
+    experts = [DevExpert(lib, pkg, "fp4", inter, hidden, dgen) for _ in range(24)]
+    idx, w = routing(np.random.default_rng(9), 500, 2, 24, zipf=0.7)
+    tbl, di, dw = table_of(experts), torch.from_numpy(idx).to(DEV), torch.from_numpy(w).to(DEV)
+    x = torch.from_numpy(bf16_rows(torch.Generator().manual_seed(5), 500, hidden)).to(DEV)
+    scales = (1.0, 3.0, 0.25, 2.0)
+    xs = [x * s for s in scales]
+    first = [torch.empty(500, hidden, device=DEV) for _ in scales]
+    again = [torch.empty(500, hidden, device=DEV) for _ in scales]
+    for i, xi in enumerate(xs):
+        for out in (first[i], again[i]):
+            lib.moe_grouped_mx_dev(out.data_ptr(), xi.data_ptr(), 500, tbl.data_ptr(), 24, di.data_ptr(),
+                                   dw.data_ptr(), 2, None, hidden, inter, 10.0)
+    torch.cuda.synchronize()
+    for a, b in zip(first, again):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 @pytest.mark.parametrize("limit", [10.0, 0.0])
 def test_mx_swiglu_clamp(lib, pkg, oracle, limit):
     """gate and up of standard deviation 25: the clamp (and its absence)
