@@ -166,6 +166,12 @@ __device__ __forceinline__ bool qmat_matches(const DSV4QMat &m, int rows, int co
     else return m.wdt == DSV4_WFP8_F32S && m.blk_r == 128 && m.blk_c == 128;
 }
 
+/* what buffer loads need of their bases */
+__device__ __forceinline__ bool dword_aligned(const DSV4QMat &m)
+{
+    return (((uintptr_t)m.w | (uintptr_t)m.s) & 3) == 0;
+}
+
 } // namespace
 
 /* ----------------------------------------------------- rows to fp16 --- */
@@ -1113,11 +1119,8 @@ __global__ __launch_bounds__(512) void k_grouped3(GroupedArgs a)
     }
     const int f0 = slab * FEAT;
     const int K = a.K, N = a.N;
-    /* buffer loads need dword-aligned weights and scales */
-    const bool aligned = (((uintptr_t)m1.w | (uintptr_t)m1.s) & 3) == 0 &&
-                         (!SWIGLU || (((uintptr_t)m3.w | (uintptr_t)m3.s) & 3) == 0);
     if (!qmat_matches<FMT_FP4_E8M0>(m1, N, K) || (SWIGLU && !qmat_matches<FMT_FP4_E8M0>(m3, N, K)) ||
-        !aligned) {
+        !dword_aligned(m1) || (SWIGLU && !dword_aligned(m3))) {
         if (threadIdx.x == 0) atomicOr(a.status, ST_BAD_DESCRIPTOR);
         const float nan = __builtin_nanf("");
         for (int i = threadIdx.x; i < ntok * FEAT; i += 64 * C::NWAVE) {
@@ -1345,7 +1348,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     const DSV4QMat m1 = SWIGLU ? e.w1 : e.w2, m3 = e.w3;
     const int f0 = slab * FEAT;
     const int K = a.K, N = a.N;
-    if (!qmat_matches<FMT_FP4_E8M0>(m1, N, K) || (SWIGLU && !qmat_matches<FMT_FP4_E8M0>(m3, N, K))) {
+    if (!qmat_matches<FMT_FP4_E8M0>(m1, N, K) || (SWIGLU && !qmat_matches<FMT_FP4_E8M0>(m3, N, K)) ||
+        !dword_aligned(m1) || (SWIGLU && !dword_aligned(m3))) {
         if (threadIdx.x == 0) atomicOr(a.status, ST_BAD_DESCRIPTOR);
         const float nan = __builtin_nanf("");
         for (int i = threadIdx.x; i < ntok * FEAT; i += 256) {

@@ -536,6 +536,22 @@ def test_grouped_dword_aligned_experts(lib, pkg, oracle, counts, hidden, inter):
     assert e <= REL_L2_TOL, f"rel L2 {e:.3e} (max abs {max_abs(got, want):.3e})"
 
 
+@pytest.mark.parametrize("counts,hidden", [([3, 0, 18], 1024), ([60] * 64, 512)])    # streaming, 128-row tiles
+@pytest.mark.parametrize("name,field,by", [("w1", "w", 2), ("w3", "s", 1), ("w2", "w", 1), ("w2", "s", 3)])
+def test_grouped_misaligned_expert_flags_status(lib, pkg, counts, hidden, name, field, by):
+    """A table whose expert weights or scales start off a 4-byte boundary
+    raises status bit 1 (value 2) and its tokens come back as NaN; no load
+    uses them."""
+    experts, x, idx, w = bucket_case(lib, pkg, counts, hidden, hidden, 17)
+    q = getattr(experts[0].desc, name)
+    setattr(q, field, getattr(q, field) - 4 + by)
+    lib.status()
+    got = run_dev(lib, experts, None, x, idx, w, hidden, hidden)
+    assert lib.status() == 2
+    hit = idx[:, 0] == 0
+    assert np.isnan(got[hit]).all() and np.isfinite(got[~hit]).all()
+
+
 @pytest.mark.parametrize("fmt", ["fp8f32", "fp8e8m0"])
 @pytest.mark.parametrize("hidden,inter,tokens", [(256, 2048, (64, 150, 193, 333, 450, 700)), (512, 640, (40, 210))])
 def test_shared_tile_sizes_same_bits(lib, pkg, oracle, hidden, inter, tokens, fmt):
