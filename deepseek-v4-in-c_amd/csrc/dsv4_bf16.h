@@ -4,6 +4,7 @@
 #ifndef DSV4_BF16_H
 #define DSV4_BF16_H
 
+#include "dsv4_choose.h"
 #include "dsv4_dev.h"
 
 namespace dsv4 {
@@ -154,10 +155,6 @@ struct Bf16Tile {
  * loads first, so the call waits out one memory latency, then every wave
  * runs four of the chains, one MFMA a step: lane i + 4 b + 16 k supplies row
  * i, token i of chain 4 b + w for wave w. */
-constexpr int B4_COLS = 4096;
-constexpr int B4_W_LD = 2 * B4_COLS + 64, B4_X_LD = 4 * B4_COLS + 16;    /* bank offsets */
-constexpr int b4_lds_bytes(int ntok) { return 4 * B4_W_LD + ntok * B4_X_LD; }
-
 /* Returns the dot product of row row0 + lane / 16 and token t0 + lane % 4 in
  * wave 0's lanes with (lane & 12) == 0. lds: b4_lds_bytes(min(ntok, 4)). Rows
  * past the end repeat the last, tokens past the end give no result. */

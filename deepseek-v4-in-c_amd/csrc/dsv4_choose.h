@@ -1,0 +1,133 @@
+/* SPDX-License-Identifier: Apache-2.0 */
+/* dsv4_choose.h - which form a call's sizes take: the rules of the dispatch as
+ * plain arithmetic on the host, with nothing of HIP, so that the CPU tests
+ * compile and ask them (tests/test_choice.py). Costs are in the unit that each
+ * rule names, rounds are of CUS workgroups. */
+#ifndef DSV4_CHOOSE_H
+#define DSV4_CHOOSE_H
+
+#include <stddef.h>
+
+namespace dsv4 {
+
+constexpr long CUS = 256;                              /* compute units of an MI355X */
+
+inline long ceil_div(long a, long b) { return (a + b - 1) / b; }
+inline long rounds(long workgroups) { return ceil_div(workgroups, CUS); }
+
+/* ---- FP8 and MXFP8 GEMMs (dsv4_gemm.hip, dsv4_gemm_mid.hip) ---- */
+
+/* The k_gemm_mid tile of 16 t tokens (t = 2, 4, 8) of least cost, 0 for the 128
+ * x 256 tiles: a round of 256 workgroups takes 11, 15 or 23 us with T = 2, 4 or
+ * 8 at 4,096 columns, of the 128 x 256 tiles 30. us of the call
+ * with T = 2 / 4 / 8 / 128 x 256, MXFP8: 4096 x 4096 300 tokens 20.2 / 18.2 /
+ * 22.7 / 30.0, 700 tokens 32.8 / 28.8 / 26.4 / 32.1, 1,500 tokens 57.6 / 46.5 /
+ * 48.1 / 38.1; 2048 x 7168 700 tokens 36.2 / 29.1 / 35.3 / 48.0. The loads
+ * address A, W and Sa with 31-bit byte offsets, and a row block's scales fit
+ * one register. */
+constexpr int GEMM_MID_KMAX = 64 * 128;
+inline int gemm_mid_tile(int M, int N, int K)
+{
+    if (M <= 0 || N % 128 || K % 128 || K > GEMM_MID_KMAX || (size_t)M * K >= (1u << 31) ||
+        (size_t)M * N / 1024 >= (1u << 31))
+        return 0;
+    const int t[3] = {2, 4, 8}, c[3] = {11, 15, 23};
+    int best = 0;
+    long cost = 30 * rounds(ceil_div(M, 128) * ceil_div(N, 256));
+    for (int i = 0; i < 3; i++) {
+        const long v = c[i] * rounds(ceil_div(M, 16 * t[i]) * (N / 128));
+        if (best ? v < cost : v <= cost) {
+            best = t[i];
+            cost = v;
+        }
+    }
+    return best;
+}
+
+/* ---- FP8 matrices over many tokens (k_dense8, the seam GEMM) ---- */
+
+/* The 16-token groups T of a k_dense8 tile with the least cost: a round of 256
+ * workgroups takes 8, 11, 16, 19 or 26 us with T = 1, 2, 3, 4 or 6 for 4,096
+ * columns (tiles smaller than their share re-read the weights, larger ones
+ * leave CUs idle). 4096 x 4096, us of the call with T = 1 / 2 / 3 / 4 / 6: 77
+ * tokens 16.5 / 19.9 / 21.9 / 23.6 / 27.3, 333 tokens 33.4 / 28.6 / 25.3 / 26.6
+ * / 30.6, 700 tokens 56.6 / 44.4 / 45.3 / 48.1 / 35.9. slabs: 128-row blocks of
+ * the matrix (gate/up: 64 rows of each). */
+inline int dense8_tile(int M, long slabs, long *cost)
+{
+    const int t[5] = {1, 2, 3, 4, 6}, c[5] = {8, 11, 16, 19, 26};
+    int best = 0;
+    for (int i = 0; i < 5; i++) {
+        const long v = c[i] * rounds(ceil_div(M, 16 * t[i]) * slabs);
+        if (!best || v < *cost) {
+            best = t[i];
+            *cost = v;
+        }
+    }
+    return best;
+}
+
+/* Whether an FP8 matrix of rows x cols against nt tokens takes the seam GEMM
+ * (128 x 256 tiles) rather than k_dense8 (dense) or, for operands that k_dense8
+ * does not address, the grouped form. The seam GEMM's round is 60 in
+ * dense8_tile's units: 4096 x 4096, 1,500 tokens 68.1 against 67.2 us dense,
+ * 2,048 tokens 77.5 / 108.8; 1024 x 4096, 2,048 tokens 65.5 / 37.6. */
+constexpr int MMQ_SEAM_GEMM_MIN_TOKENS = 1280;
+inline bool mmq_takes_seam(int nt, int rows, bool dense)
+{
+    if (!dense) return nt >= MMQ_SEAM_GEMM_MIN_TOKENS;
+    long cost = 0;
+    dense8_tile(nt, rows / 128, &cost);
+    return 60 * rounds(ceil_div(nt, 128) * ceil_div(rows, 256)) < cost;
+}
+
+/* ---- routed FP4 experts (dsv4_moe_grouped.hip) ---- */
+
+/* Tiles of the grouped GEMMs: 1, 4 or 8 times 16 rows, the 16-row tiles that
+ * stream the weights to registers, or the dense tiles of one FP8 matrix. */
+constexpr int GROUPED_STREAM = 5, GROUPED_DENSE = 6;
+
+/* The form of the routed experts' GEMMs, by the mean bucket. Up to 28 rows an
+ * expert the weight stream is the bound: the 16-row tiles that stream to
+ * registers (4096 x 2048, 256 experts: 7 tokens 135 against 161 us of the
+ * LDS-staged 16-row tiles, 64 tokens 297 / 356, 701 tokens 870 / 1,005 and
+ * 1,128 of the 128-row tiles; at 33 rows an expert 1,233 / 1,374 / 1,193).
+ * With fewer than four steps of 256 to a row its setup costs more than it
+ * saves (inter 512: 62 against 59 us at 60 tokens): there the LDS-staged
+ * tiles, 16 rows up to 16 rows an expert, else 128 rows (weights reused
+ * across a tile; 64 experts, hidden 4096, inter 512: 60 tokens 89 against 101
+ * us, 300 tokens 146 / 134, 700 tokens 223 / 187). stream: the geometry is one
+ * that the streaming tiles take. */
+inline int grouped_form(long pairs, int n_experts, int hidden, int inter, bool stream)
+{
+    if (pairs <= 28L * n_experts && hidden >= 1024 && inter >= 1024 && stream) return GROUPED_STREAM;
+    return pairs <= 16L * n_experts ? 1 : 8;
+}
+
+/* ---- BF16 matvecs (dsv4_gemv.hip) ---- */
+
+/* LDS of k_gemv4_bf16: four rows and up to four tokens, 4,096 columns at a
+ * time, a bank offset behind each. */
+constexpr int B4_COLS = 4096;
+constexpr int B4_W_LD = 2 * B4_COLS + 64, B4_X_LD = 4 * B4_COLS + 16;
+constexpr int b4_lds_bytes(int ntok) { return 4 * B4_W_LD + ntok * B4_X_LD; }
+
+/* Which form, all with the same bits. us at 4096 columns for (small /
+ * rows / GEMM), measured: 1 token: 1024 rows 6.4 / 20 / 15, 8192 rows 18.8 /
+ * 22 / 25, 16384 rows 37 / 25 / 45; 4 tokens: 256 rows 6.7 / - / 15, 4096
+ * rows 20 / 31 / 16, 8192 rows 37 / 31 / 26, 32768 rows 147 / 61 / 88; 32
+ * tokens: 256 rows 10.1 / - / 15, 1024 rows 36 / - / 15. So: the rows form
+ * for a few tokens of a large matrix, the small form while its workgroups
+ * run in at most three rounds of what LDS lets the device hold at once, else
+ * the GEMM. */
+enum Bf16Form { BF16_SMALL = 1, BF16_ROWS, BF16_GEMM };
+inline Bf16Form bf16_form(int rows, int nt)
+{
+    if (nt <= 4 && rows >= (nt == 1 ? 9216 : 12288)) return BF16_ROWS;
+    const int lds = b4_lds_bytes(nt < 4 ? nt : 4);
+    return ceil_div(rows, 4) * ceil_div(nt, 4) <= 3 * CUS * (160 * 1024 / lds) ? BF16_SMALL : BF16_GEMM;
+}
+
+} // namespace dsv4
+
+#endif /* DSV4_CHOOSE_H */

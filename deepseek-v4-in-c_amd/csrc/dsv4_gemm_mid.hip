@@ -41,7 +41,7 @@ typedef __attribute__((address_space(3))) void lds_void;
 enum { T_FP8 = 0, T_MX = 1 };
 
 constexpr int TB = 128;                            /* reduction block           */
-constexpr int T_KMAX = 64 * TB;
+static_assert(GEMM_MID_KMAX == 64 * TB, "one lane to a weight scale");
 constexpr uint32_t T_OOB = 0x80000000u;            /* beyond every buffer       */
 constexpr int T_E8M0_ONE = 127;
 
@@ -291,30 +291,6 @@ hipError_t gemm_mid_fp8_launch(const GemmArgs &g, bool w_f32s, bool out_bf16, in
 hipError_t gemm_mid_mx_launch(const GemmArgs &g, bool out_bf16, int t, hipStream_t st)
 {
     return mid_t<T_MX, false>(mid_args(g), out_bf16, t, st);
-}
-
-/* The tile of least cost: a round of 256 workgroups takes 11, 15 or 23 us with
- * T = 2, 4 or 8 at 4,096 columns, of the 128 x 256 tiles 30. us of the call
- * with T = 2 / 4 / 8 / 128 x 256, MXFP8: 4096 x 4096 300 tokens 20.2 / 18.2 /
- * 22.7 / 30.0, 700 tokens 32.8 / 28.8 / 26.4 / 32.1, 1,500 tokens 57.6 / 46.5 /
- * 48.1 / 38.1; 2048 x 7168 700 tokens 36.2 / 29.1 / 35.3 / 48.0. The loads
- * address A, W and Sa with 31-bit byte offsets, and a row block's scales fit
- * one register. */
-int gemm_mid_tile(int M, int N, int K)
-{
-    if (M <= 0 || N % 128 || K % TB || K > T_KMAX || (size_t)M * K >= (1u << 31) || (size_t)M * N / 1024 >= (1u << 31))
-        return 0;
-    const int t[3] = {2, 4, 8}, c[3] = {11, 15, 23};
-    int best = 0;
-    long cost = 30 * (((M + 127L) / 128 * ((N + 255) / 256) + 255) / 256);
-    for (int i = 0; i < 3; i++) {
-        const long v = c[i] * ((((long)M + 16 * t[i] - 1) / (16 * t[i]) * (N / 128) + 255) / 256);
-        if (best ? v < cost : v <= cost) {
-            best = t[i];
-            cost = v;
-        }
-    }
-    return best;
 }
 
 } // namespace dsv4

@@ -253,26 +253,17 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemvBf16Args a)
     a.y[(size_t)(t0 + lr) * a.y_ld + r0 + row] = (float)v;
 }
 
-/* Which form, all three with the same bits. us at 4096 columns for (small /
- * rows / GEMM), measured: 1 token: 1024 rows 6.4 / 20 / 15, 8192 rows 18.8 /
- * 22 / 25, 16384 rows 37 / 25 / 45; 4 tokens: 256 rows 6.7 / - / 15, 4096
- * rows 20 / 31 / 16, 8192 rows 37 / 31 / 26, 32768 rows 147 / 61 / 88; 32
- * tokens: 256 rows 10.1 / - / 15, 1024 rows 36 / - / 15. So: the rows form
- * for a few tokens of a large matrix, the small form while its workgroups
- * run in at most three rounds of what LDS lets the device hold at once, else
- * the GEMM. */
 hipError_t gemv_bf16_launch(const GemvBf16Args &a, hipStream_t st)
 {
     if (a.rows <= 0 || a.cols <= 0 || a.cols % 8 || a.nt <= 0) return hipErrorInvalidValue;
-    if (a.nt <= 4 && a.rows >= (a.nt == 1 ? 9216 : 12288)) {
+    const Bf16Form form = bf16_form(a.rows, a.nt);
+    if (form == BF16_ROWS) {
         constexpr int RG = 2;
         const int waves = (a.rows + 8 * RG - 1) / (8 * RG);
         hipLaunchKernelGGL((k_gemv_bf16<RG, 8>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, a);
         return hipGetLastError();
     }
-    const int lds = b4_lds_bytes(a.nt < 4 ? a.nt : 4);
-    const long small = (((long)a.rows + 3) / 4) * (((long)a.nt + 3) / 4);
-    if (small <= 3L * 256 * (160 * 1024 / lds)) {
+    if (form == BF16_SMALL) {
         static bool attr_done = false;             /* not again inside a stream capture of a later call */
         if (!attr_done) {
             const hipError_t e = hipFuncSetAttribute((const void *)k_gemv4_bf16,
@@ -281,7 +272,7 @@ hipError_t gemv_bf16_launch(const GemvBf16Args &a, hipStream_t st)
             attr_done = true;
         }
         hipLaunchKernelGGL(k_gemv4_bf16, dim3((unsigned)((a.rows + 3) / 4), (unsigned)((a.nt + 3) / 4)), dim3(256),
-                           lds, st, a);
+                           b4_lds_bytes(a.nt < 4 ? a.nt : 4), st, a);
         return hipGetLastError();
     }
     const long grid = (((long)a.nt + 15) / 16) * (((long)a.rows + 15) / 16);

@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "../../include/dsv4_hip.h"
+#include "dsv4_choose.h"
 #include "dsv4_dev.h"
 
 namespace dsv4 {
@@ -334,9 +335,7 @@ bool gemm_seam_ok(int M, int N, int K);
 hipError_t gemm_seam_launch(const SeamGemmArgs &s, bool w_f32s, hipStream_t st);
 
 /* The FP8 and MXFP8 GEMMs in tiles of 128 features x 16 t tokens
- * (dsv4_gemm_mid.hip); gemm_mid_tile: the t a shape takes, 0 for the large
- * tiles. */
-int gemm_mid_tile(int M, int N, int K);
+ * (dsv4_gemm_mid.hip), t as gemm_mid_tile gives it. */
 hipError_t gemm_mid_fp8_launch(const GemmArgs &g, bool w_f32s, bool out_bf16, int t, hipStream_t st);
 hipError_t gemm_mid_mx_launch(const GemmArgs &g, bool out_bf16, int t, hipStream_t st);
 
@@ -479,14 +478,11 @@ struct GroupedArgs {
 };
 /* tt: 1 or 4 (16- or 64-row tiles), 8 (128-row, FP4), GROUPED_STREAM (16-row,
  * FP4 experts of a table, geometry as grouped_stream_ok) or GROUPED_DENSE (one
- * FP8 matrix, operands as grouped_dense_cost) */
-constexpr int GROUPED_STREAM = 5, GROUPED_DENSE = 6;
+ * FP8 matrix, operands as grouped_dense_ok) */
 int grouped_rows_per_tile(int tt);
 bool grouped_stream_ok(long nrows, int K, int N);
-/* the cost of the GROUPED_DENSE form, in the units of GROUPED_DENSE_SEAM per
- * round of 256 workgroups of the seam GEMM; 0: it does not take the operands */
-constexpr long GROUPED_DENSE_SEAM = 60;
-long grouped_dense_cost(const GroupedArgs &a, int fmt, bool swiglu);
+/* whether the GROUPED_DENSE form takes the operands */
+bool grouped_dense_ok(const GroupedArgs &a, int fmt, bool swiglu);
 hipError_t grouped_launch(int fmt, bool swiglu, int tt, const GroupedArgs &a, long max_tiles,
                           hipStream_t st);
 

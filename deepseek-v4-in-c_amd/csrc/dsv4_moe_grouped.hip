@@ -1830,42 +1830,18 @@ static hipError_t dense8_t(const GroupedArgs &a, hipStream_t st)
     return hipGetLastError();
 }
 
-/* The 16-token groups T of a k_dense8 tile with the least cost: a round of 256
- * workgroups takes 8, 11, 16, 19 or 26 us with T = 1, 2, 3, 4 or 6 for 4,096
- * columns (tiles smaller than their share re-read the weights, larger ones
- * leave CUs idle). 4096 x 4096, us of the call with T = 1 / 2 / 3 / 4 / 6: 77
- * tokens 16.5 / 19.9 / 21.9 / 23.6 / 27.3, 333 tokens 33.4 / 28.6 / 25.3 / 26.6
- * / 30.6, 700 tokens 56.6 / 44.4 / 45.3 / 48.1 / 35.9. */
-static int dense8_tile(int M, long slabs, long *cost)
-{
-    const int t[5] = {1, 2, 3, 4, 6}, c[5] = {8, 11, 16, 19, 26};
-    int best = 0;
-    for (int i = 0; i < 5; i++) {
-        const long v = c[i] * ((((long)M + 16 * t[i] - 1) / (16 * t[i]) * slabs + 255) / 256);
-        if (!best || v < *cost) {
-            best = t[i];
-            *cost = v;
-        }
-    }
-    return best;
-}
-
 /* k_dense8 takes rows of up to its scale register's 64 blocks, weights on
  * 16-byte boundaries and 31-bit offsets; what its callers' other forms flag
  * in the kernel goes to those. */
-long grouped_dense_cost(const GroupedArgs &a, int fmt, bool swiglu)
+bool grouped_dense_ok(const GroupedArgs &a, int fmt, bool swiglu)
 {
     auto ok = [&](const DSV4QMat &m) {
         return m.rows == a.N && m.cols == a.K && m.w && m.s && ((uintptr_t)m.w & 15) == 0 && m.blk_r == 128 &&
                m.blk_c == 128 && m.wdt == (fmt == FMT_FP8_F32S ? DSV4_WFP8_F32S : DSV4_WFP8);
     };
-    if (a.table || (fmt != FMT_FP8_E8M0 && fmt != FMT_FP8_F32S) || a.K % KC || a.K > D8_KMAX || a.N % 128 ||
-        a.nrows <= 0 || !ok(a.m1) || (swiglu && !ok(a.m3)) || (size_t)a.nrows * a.K * 2 >= (1u << 31) ||
-        (size_t)a.N * a.K >= (1u << 31))
-        return 0;
-    long cost = 0;
-    dense8_tile(a.nrows, a.N / (swiglu ? 64 : 128), &cost);
-    return cost;
+    return !a.table && (fmt == FMT_FP8_E8M0 || fmt == FMT_FP8_F32S) && a.K % KC == 0 && a.K <= D8_KMAX &&
+           a.N % 128 == 0 && a.nrows > 0 && ok(a.m1) && (!swiglu || ok(a.m3)) &&
+           (size_t)a.nrows * a.K * 2 < (1u << 31) && (size_t)a.N * a.K < (1u << 31);
 }
 
 template <bool WS, bool SW>
@@ -1937,7 +1913,7 @@ hipError_t grouped_launch(int fmt, bool swiglu, int tt, const GroupedArgs &a, lo
         return swiglu ? grouped_w<true>(a, items, st) : grouped_w<false>(a, items, st);
     }
     if (tt == GROUPED_DENSE) {
-        if (!grouped_dense_cost(a, fmt, swiglu)) return hipErrorInvalidValue;
+        if (!grouped_dense_ok(a, fmt, swiglu)) return hipErrorInvalidValue;
         if (fmt == FMT_FP8_F32S) return swiglu ? dense8<true, true>(a, st) : dense8<true, false>(a, st);
         return swiglu ? dense8<false, true>(a, st) : dense8<false, false>(a, st);
     }

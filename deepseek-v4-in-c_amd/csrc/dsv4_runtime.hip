@@ -764,17 +764,13 @@ void *dsv4_hip_device_ptr(const void *p)
  * kernel takes (rows, cols multiples of 128; FP8 with 128x128 blocks or FP4
  * with 1x32) run as one dense fp16-MFMA GEMM (x row-scaled by a power of two
  * and rounded to fp16, weights decoded exactly, fp32 accumulation), FP8 by
- * cost in the dense tiles (k_dense8) or the GEMM-shaped seam kernel (128 x 256
- * tiles, about 60 us a round of 256 at 4,096 columns: 4096 x 4096, 1,500
- * tokens 68.1 against 67.2 us dense, 2,048 tokens 77.5 / 108.8; 1024 x 4096,
- * 2,048 tokens 65.5 / 37.6), FP4 and rows the dense tiles do not take in the
- * grouped kernel with one group (the same bits in all three; the seam kernel
- * from MMQ_SEAM_GEMM_MIN_TOKENS there, 4096 x 4096: 64 us from 128 to 1,024
- * tokens, 79 at 2,048, the grouped form 59 at 1,024, 82 at 1,536); fewer
- * tokens run the block-scaled MFMA GEMV where its geometry fits, else the
- * per-token VALU GEMV. */
+ * cost in the dense tiles (k_dense8) or the GEMM-shaped seam kernel
+ * (mmq_takes_seam), FP4 and matrices of 2 GiB and more in the grouped kernel
+ * with one group (the same bits in all three). Fewer tokens run the
+ * block-scaled MFMA GEMV where its geometry fits, else the per-token VALU
+ * GEMV. FP8 rows past 8,192 bytes and other blocks never get here: they are
+ * the generic matvec's. */
 constexpr int MMQ_MFMA_MIN_TOKENS = 32;
-constexpr int MMQ_SEAM_GEMM_MIN_TOKENS = 1280;
 /* From this many tokens the block-scaled MFMA GEMV splits x once into its
  * e4m3 part tables (k_split_x_tab) and walks the token groups with each row
  * block's weights held (k_gemv_mx_tab), rather than every row block
@@ -811,9 +807,8 @@ static int enqueue_mmq(const DSV4QMat &d, int fmt, const float *x, float *y, int
         memset(&a, 0, sizeof a);
         a.m1 = d; a.nrows = nt; a.B = x16; a.bexp = ex; a.K = d.cols; a.N = d.rows; a.out = y;
         a.status = g.st;
-        const long dense = grouped_dense_cost(a, fmt, false);
-        const long seam = GROUPED_DENSE_SEAM * (((nt + 127L) / 128 * ((d.rows + 255) / 256) + 255) / 256);
-        if (fmt != FMT_FP4_E8M0 && (dense ? seam < dense : nt >= MMQ_SEAM_GEMM_MIN_TOKENS) && aligned16(d.w) &&
+        const bool dense = grouped_dense_ok(a, fmt, false);
+        if (fmt != FMT_FP4_E8M0 && mmq_takes_seam(nt, d.rows, dense) && aligned16(d.w) &&
             gemm_seam_ok(nt, d.rows, d.cols)) {
             SeamGemmArgs sg;
             sg.X = x16; sg.ex = ex; sg.W = (const uint8_t *)d.w; sg.Sw = d.s; sg.C = y;
@@ -825,10 +820,9 @@ static int enqueue_mmq(const DSV4QMat &d, int fmt, const float *x, float *y, int
             HIPCHK(grouped_launch(fmt, false, GROUPED_DENSE, a, 1, st), "dense MFMA launch");
             return 0;
         }
-        /* 16-token tiles give a small batch more workgroups (4096 x 4096
-         * FP8: 23 us from 32 to 128 tokens, against 28-32 us in 64-token
-         * tiles), 64-token tiles reuse each weight chunk more from about 200
-         * tokens on (256 tokens: 33 against 37 us) */
+        /* 16-token tiles give a small batch more workgroups, 64-token tiles
+         * reuse each weight chunk more (4096 x 4096: 32 to 128 tokens 23 us
+         * against 28-32 in 64-token tiles, 256 tokens 37 against 33) */
         const int tt = nt <= 192 ? 1 : 4;
         const long tiles = (nt + grouped_rows_per_tile(tt) - 1) / grouped_rows_per_tile(tt);
         HIPCHK(grouped_launch(fmt, false, tt, a, tiles, st), "dense MFMA launch");
@@ -1554,24 +1548,6 @@ int dsv4_hip_gemm_mxfp8q_dev(void *C, int out_bf16, const uint8_t *Aq, const uin
 
 /* ------------------------------------------------------ grouped MoE --- */
 
-/* The form of the routed experts' GEMMs, by the mean bucket. Up to 28 rows an
- * expert the weight stream is the bound: the 16-row tiles that stream to
- * registers (4096 x 2048, 256 experts: 7 tokens 135 against 161 us of the
- * LDS-staged 16-row tiles, 64 tokens 297 / 356, 701 tokens 870 / 1,005 and
- * 1,128 of the 128-row tiles; at 33 rows an expert 1,233 / 1,374 / 1,193).
- * With fewer than four steps of 256 to a row its setup costs more than it
- * saves (inter 512: 62 against 59 us at 60 tokens): there the LDS-staged
- * tiles, 16 rows up to 16 rows an expert, else 128 rows (weights reused
- * across a tile; 64 experts, hidden 4096, inter 512: 60 tokens 89 against 101
- * us, 300 tokens 146 / 134, 700 tokens 223 / 187). */
-static int grouped_tt(long pairs, int n_experts, int n, int hidden, int inter)
-{
-    if (pairs <= 28L * n_experts && hidden >= 1024 && inter >= 1024 && grouped_stream_ok(n, hidden, inter) &&
-        grouped_stream_ok(pairs, inter, hidden))
-        return GROUPED_STREAM;
-    return pairs <= 16L * n_experts ? 1 : 8;
-}
-
 /* A shared expert's matrix beside the routed ones: an FP8 one over many tokens
  * in the dense tiles (701 tokens, the call: 890 -> 846 us, 2,048: 1,546 ->
  * 1,454; up to 192 the 16- and 64-row tiles disturb the routed launches less:
@@ -1579,7 +1555,7 @@ static int grouped_tt(long pairs, int n_experts, int n, int hidden, int inter)
 static int enqueue_dense(int fmt, bool swiglu, const GroupedArgs &a, hipStream_t st, const char *what)
 {
     int tt = a.nrows <= 64 ? 1 : 4;          /* enough workgroups for a small batch */
-    if (a.nrows > 192 && grouped_dense_cost(a, fmt, swiglu)) tt = GROUPED_DENSE;
+    if (a.nrows > 192 && grouped_dense_ok(a, fmt, swiglu)) tt = GROUPED_DENSE;
     const long rows = tt == GROUPED_DENSE ? a.nrows : grouped_rows_per_tile(tt);
     HIPCHK(grouped_launch(fmt, swiglu, tt, a, (a.nrows + rows - 1) / rows, st), what);
     return 0;
@@ -1591,7 +1567,8 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
                         int inter, float limit, hipStream_t st, bool forked)
 {
     const long P = (long)n * topk;
-    int tt = grouped_tt(P, n_experts, n, hidden, inter);
+    int tt = grouped_form(P, n_experts, hidden, inter,
+                          grouped_stream_ok(n, hidden, inter) && grouped_stream_ok(P, inter, hidden));
     /* the 128-row kernel takes 256 down rows per workgroup and 31-bit offsets */
     if (tt == 8 && (hidden % 256 || (size_t)P * inter * 2 >= (1u << 31) ||
                     (size_t)n * hidden * 2 >= (1u << 31) || (size_t)inter * hidden / 2 >= (1u << 31)))

@@ -1,0 +1,67 @@
+# SPDX-License-Identifier: Apache-2.0
+"""The rules that pick a kernel by a call's sizes (csrc/dsv4_choose.h),
+compiled for the host: the forms that were measured to be the faster ones, and
+the forms that the GPU tests of the kernels rely on reaching."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+from conftest import PKG_DIR
+
+SHIM = """
+#include "dsv4_choose.h"
+using namespace dsv4;
+extern "C" {
+int c_gemm_mid_tile(int M, int N, int K) { return gemm_mid_tile(M, N, K); }
+int c_dense8_tile(int M, long slabs) { long c = 0; return dense8_tile(M, slabs, &c); }
+int c_mmq_takes_seam(int nt, int rows, int dense) { return mmq_takes_seam(nt, rows, dense != 0); }
+int c_grouped_form(long pairs, int ne, int hidden, int inter, int stream)
+{ return grouped_form(pairs, ne, hidden, inter, stream != 0); }
+int c_bf16_form(int rows, int nt) { return bf16_form(rows, nt); }
+}
+"""
+STREAM = 5
+SMALL, ROWS, GEMM = 1, 2, 3
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("choice")
+    src, so = d / "shim.cpp", d / "shim.so"
+    src.write_text(SHIM)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I",
+                    os.path.join(PKG_DIR, "csrc"), str(src), "-o", str(so)], check=True)
+    lib = C.CDLL(str(so))
+    lib.c_dense8_tile.argtypes = [C.c_int, C.c_long]
+    lib.c_grouped_form.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int]
+    return lib
+
+
+@pytest.mark.parametrize("tokens,rows,cols,tile", [
+    (8, 1024, 4096, 2), (300, 1024, 4096, 2), (300, 4096, 4096, 4), (700, 4096, 4096, 8), (1500, 4096, 4096, 0),
+    (300, 1024, 8320, 0),                                  # more weight scales than a register holds
+])
+def test_gemm_tile(rules, tokens, rows, cols, tile):
+    assert rules.c_gemm_mid_tile(tokens, rows, cols) == tile
+
+
+@pytest.mark.parametrize("tokens,rows,tile", [(77, 4096, 1), (333, 4096, 3), (700, 4096, 6)])
+def test_dense_tile(rules, tokens, rows, tile):
+    assert rules.c_dense8_tile(tokens, rows // 128) == tile
+
+
+@pytest.mark.parametrize("tokens,experts,hidden,inter,form", [
+    (7, 256, 4096, 2048, STREAM), (64, 256, 4096, 2048, STREAM), (701, 256, 4096, 2048, STREAM),
+    (1500, 256, 4096, 2048, 8), (60, 64, 4096, 512, 1), (700, 64, 4096, 512, 8),
+])
+def test_expert_tiles_top6(rules, tokens, experts, hidden, inter, form):
+    assert rules.c_grouped_form(6 * tokens, experts, hidden, inter, 1) == form
+
+
+@pytest.mark.parametrize("rows,tokens,form", [
+    (256, 1, SMALL), (256, 8, SMALL), (129280, 1, ROWS), (16384, 4, ROWS), (4096, 4, GEMM), (256, 700, GEMM),
+])
+def test_bf16_form(rules, rows, tokens, form):
+    assert rules.c_bf16_form(rows, tokens) == form
