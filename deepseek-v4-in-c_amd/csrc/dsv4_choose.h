@@ -97,11 +97,29 @@ constexpr int GROUPED_STREAM = 5, GROUPED_DENSE = 6;
  * tiles, 16 rows up to 16 rows an expert, else 128 rows (weights reused
  * across a tile; 64 experts, hidden 4096, inter 512: 60 tokens 89 against 101
  * us, 300 tokens 146 / 134, 700 tokens 223 / 187). stream: the geometry is one
- * that the streaming tiles take. */
+ * that the streaming tiles take.
+ *
+ * Few experts make few 128-row tiles, and a workgroup of those takes its time
+ * however many CUs stay idle: up to 4,096 pairs, where they do not fill the
+ * device once, they have to be the cheaper ones (us of 16 / 128 rows, hidden
+ * 4096, inter 2048: one expert, 100 tokens 36 / 85, 560 tokens 84 / 98, 1,600
+ * tokens 194 / 131; eight experts, 140 rows each, 138 / 106; 2048 x 512, one
+ * expert, 800 tokens 36 / 59). In units of a 16-row tile's multiplications, one
+ * per weight: a 128-row workgroup's latency grows with its K and, by 0.3 + 0.7
+ * rows / 128, with the tile's rows; 45 and 1.5 fit 390 measured calls of 1 to 64
+ * experts (7168 x 2048 to 512 x 512) within 10 % of the better form. */
+constexpr long GROUPED_FEW_PAIRS = 4096;
 inline int grouped_form(long pairs, int n_experts, int hidden, int inter, bool stream)
 {
-    if (pairs <= 28L * n_experts && hidden >= 1024 && inter >= 1024 && stream) return GROUPED_STREAM;
-    return pairs <= 16L * n_experts ? 1 : 8;
+    const int form16 = stream && hidden >= 1024 && inter >= 1024 ? GROUPED_STREAM : 1;
+    if (pairs <= (form16 == GROUPED_STREAM ? 28L : 16L) * n_experts) return form16;
+    const double buckets = (double)(pairs < n_experts ? pairs : n_experts), rows = (double)pairs / buckets;
+    const double tiles16 = (double)pairs / 16 + buckets / 2;
+    const double tiles128 = rows > 64 ? (double)pairs / 128 + buckets / 2 : buckets;
+    if (pairs > GROUPED_FEW_PAIRS || tiles128 * inter / 128 >= (double)CUS) return 8;
+    const double weights = (double)hidden * inter;
+    const double latency = 45.0 * 1024.0 * (hidden + inter) * (0.3 + 0.7 * (rows < 128 ? rows / 128 : 1.0));
+    return latency + 1.5 * tiles128 * weights < tiles16 * weights ? 8 : form16;
 }
 
 /* ---- BF16 matvecs (dsv4_gemv.hip) ---- */

@@ -60,6 +60,19 @@ def test_expert_tiles_top6(rules, tokens, experts, hidden, inter, form):
     assert rules.c_grouped_form(6 * tokens, experts, hidden, inter, 1) == form
 
 
+@pytest.mark.parametrize("pairs,experts,hidden,inter,form", [
+    (50, 1, 4096, 2048, STREAM), (400, 1, 4096, 2048, STREAM), (200, 2, 4096, 2048, STREAM), (400, 4, 4096, 2048, STREAM),
+    (1600, 1, 4096, 2048, 8), (1120, 8, 4096, 2048, 8), (3200, 16, 4096, 2048, 8),
+    (100, 1, 2048, 512, 1), (800, 1, 2048, 512, 1), (400, 8, 2048, 512, 1), (800, 2, 512, 512, 1),
+    (4097, 1, 512, 512, 8),                                # past GROUPED_FEW_PAIRS
+    (3200, 64, 4096, 2048, 8), (2240, 32, 2048, 512, 8),   # tiles enough for every CU
+])
+def test_expert_tiles_few_experts(rules, pairs, experts, hidden, inter, form):
+    """A few experts' 128-row tiles leave the device idle: 16-row tiles until
+    there are pairs enough."""
+    assert rules.c_grouped_form(pairs, experts, hidden, inter, 1) == form
+
+
 @pytest.mark.parametrize("rows,tokens,form", [
     (256, 1, SMALL), (256, 8, SMALL), (129280, 1, ROWS), (16384, 4, ROWS), (4096, 4, GEMM), (256, 700, GEMM),
 ])

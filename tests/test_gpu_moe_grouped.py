@@ -513,7 +513,8 @@ def test_grouped_stream_scale_range_flag(lib, pkg, mat, at):
 @pytest.mark.parametrize("counts,hidden,inter", [
     ([3, 0, 18], 1024, 1024),                    # streaming tiles
     ([3, 18], 512, 512),                         # LDS-staged 16-row tiles
-    ([40, 30], 512, 512),                        # 128-row tiles
+    ([40, 30], 512, 512),                        # the same
+    ([45] * 64, 512, 512),                       # 128-row tiles
 ])
 def test_grouped_dword_aligned_experts(lib, pkg, oracle, counts, hidden, inter):
     """Expert weights and scales that start on a 4-byte boundary only."""
