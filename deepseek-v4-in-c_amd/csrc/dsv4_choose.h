@@ -122,6 +122,21 @@ inline int grouped_form(long pairs, int n_experts, int hidden, int inter, bool s
     return latency + 1.5 * tiles128 * weights < tiles16 * weights ? 8 : form16;
 }
 
+/* The mean bucket says nothing about tokens that gather on few experts, whose
+ * weights the 16-row tiles would read and decode once per 16 of them: above
+ * GROUPED_FEW_PAIRS pairs the buckets of more than GROUPED_FAT_MIN rows go to
+ * 128-row tiles in launches of their own, ahead of the others on the stream
+ * (where there are none, two launches of empty workgroups: 701 tokens, even
+ * routing, 765 -> 769 us). 256 experts of 4096 x 2048, top-6, us without / with:
+ * 1,000 tokens on 8 of them 578 / 359, on 64 660 / 435, Zipf 974 / 883; 701
+ * tokens, Zipf, 819 / 784. Fat from 96 rows: 64 experts used 586, Zipf 880; the
+ * others on a second stream beside them: Zipf 863, even routing 962 against
+ * 955. Below, 16-row tiles alone are no slower (680 tokens on 8 experts: 390). */
+constexpr int GROUPED_FAT_ROWS = 128, GROUPED_FAT_MIN = 64;
+inline bool grouped_splits(long pairs, int form) { return pairs > GROUPED_FEW_PAIRS && form != 8; }
+/* their number at most: such a bucket's tiles hold 64.5 rows each or more */
+inline long grouped_fat_tiles(long pairs) { return 2 * pairs / (GROUPED_FAT_ROWS + 1); }
+
 /* ---- BF16 matvecs (dsv4_gemv.hip) ---- */
 
 /* LDS of k_gemv4_bf16: four rows and up to four tokens, 4,096 columns at a

@@ -377,8 +377,14 @@ struct RouteArgs {
     const int *idx;           /* device [npairs]                          */
     int npairs, topk, n_experts;
     int tile_rows;            /* rows per tile of the grouped GEMM        */
+    /* fat_rows > 0: buckets of more than fat_min rows are cut into tiles of
+     * fat_rows instead, their records from tile_rec[fat_base] on, their number
+     * in tile_pre[n_experts + 1]; fewer than 65,536 of the other tiles and
+     * 32,768 of these */
+    int fat_rows = 0, fat_min = 0, fat_base = 0;
     int *grp_off;             /* [n_experts + 1] first row of each bucket */
-    int *tile_pre;            /* [n_experts + 1] prefix of tiles          */
+    int *tile_pre;            /* [n_experts + 1] prefix of tiles (one more
+                                 word with fat_rows)                      */
     TileRec *tile_rec;        /* [tiles] bucket, first row, rows per tile */
     int *pos;                 /* [npairs] row of each pair (-1: bad id)   */
     int *row_tok;             /* [npairs] token of each row               */

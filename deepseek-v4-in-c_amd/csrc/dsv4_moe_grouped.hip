@@ -300,7 +300,7 @@ __global__ __launch_bounds__(1024) void k_moe_route_count(RouteArgs a, int nch, 
  * (two launches); without, every workgroup counts every pair itself (one
  * launch, no workgroup waits for another: the form for a few chunks).
  * Workgroup 0 also writes grp_off and tile_pre, every workgroup a share
- * of the tile records; bad ids are
+ * of the tile records (with a.fat_rows two lists of them); bad ids are
  * reported by workgroup 0 (one launch) or by the counting pass. The
  * workgroups from nblk on convert a row of x each (one launch). */
 template <bool PRECOUNT>
@@ -369,7 +369,9 @@ __global__ __launch_bounds__(1024) void k_moe_route(RouteArgs a, int cpb, int nb
      * thread (E <= 1024): within each wave by shuffles, then the totals of
      * the lower waves added (two barriers) */
     const int cnt = tid < E ? hist[tid] : 0;
-    const int tls = (cnt + a.tile_rows - 1) / a.tile_rows;
+    const bool fat = a.fat_rows && cnt > a.fat_min;
+    const int rows = fat ? a.fat_rows : a.tile_rows;
+    const int tls = (cnt + rows - 1) / rows << (fat ? 16 : 0);
     {
         /* only the waves that hold experts scan (E / 64 rounded up) */
         __shared__ int wsum[2][16];
@@ -402,32 +404,39 @@ __global__ __launch_bounds__(1024) void k_moe_route(RouteArgs a, int cpb, int nb
     }
     /* each tile's bucket: the first expert whose inclusive tile prefix
      * exceeds it, tiles spread over every workgroup's threads; with the
-     * bucket's first row and the tile's rows */
-    for (int t = blockIdx.x * 1024 + tid; t < scan_t[E - 1]; t += nblk * 1024) {
+     * bucket's first row and the tile's rows. With fat_rows the upper half
+     * words count the tiles of the large buckets, which follow the others. */
+    const int fat_shift = a.fat_rows ? 16 : 0, thin_mask = a.fat_rows ? 0xFFFF : -1;
+    const int nthin = scan_t[E - 1] & thin_mask, nfat = a.fat_rows ? scan_t[E - 1] >> 16 : 0;
+    for (int i = blockIdx.x * 1024 + tid; i < nthin + nfat; i += nblk * 1024) {
+        const bool f = i >= nthin;
+        const int t = f ? i - nthin : i, trows = f ? a.fat_rows : a.tile_rows;
+        const int shift = f ? fat_shift : 0, mask = f ? 0xFFFF : thin_mask;
         int lo = 0, hi = E - 1;
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
-            if (scan_t[mid] > t) hi = mid;
+            if (((scan_t[mid] >> shift) & mask) > t) hi = mid;
             else lo = mid + 1;
         }
-        const int go = lo > 0 ? scan_r[lo - 1] : 0, tp = lo > 0 ? scan_t[lo - 1] : 0;
-        const int r0 = go + (t - tp) * a.tile_rows;
+        const int go = lo > 0 ? scan_r[lo - 1] : 0, tp = lo > 0 ? (scan_t[lo - 1] >> shift) & mask : 0;
+        const int r0 = go + (t - tp) * trows;
         TileRec rec;
         rec.grp = lo;
         rec.r0 = r0;
-        rec.ntok = min(a.tile_rows, scan_r[lo] - r0);
+        rec.ntok = min(trows, scan_r[lo] - r0);
         rec.bucket = scan_r[lo] - go;
-        a.tile_rec[t] = rec;
+        a.tile_rec[f ? a.fat_base + t : t] = rec;
     }
     if (tid < E) {
         const int o = scan_r[tid] - cnt;
         cur[tid] = o + before[tid];
         if (blockIdx.x == 0) {
             a.grp_off[tid] = o;
-            a.tile_pre[tid] = scan_t[tid] - tls;
+            a.tile_pre[tid] = (scan_t[tid] - tls) & thin_mask;
             if (tid == E - 1) {
                 a.grp_off[E] = scan_r[tid];
-                a.tile_pre[E] = scan_t[tid];
+                a.tile_pre[E] = nthin;
+                if (a.fat_rows) a.tile_pre[E + 1] = nfat;
             }
         }
     }

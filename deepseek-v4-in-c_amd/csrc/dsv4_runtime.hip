@@ -1570,16 +1570,18 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     int tt = grouped_form(P, n_experts, hidden, inter,
                           grouped_stream_ok(n, hidden, inter) && grouped_stream_ok(P, inter, hidden));
     /* the 128-row kernel takes 256 down rows per workgroup and 31-bit offsets */
-    if (tt == 8 && (hidden % 256 || (size_t)P * inter * 2 >= (1u << 31) ||
-                    (size_t)n * hidden * 2 >= (1u << 31) || (size_t)inter * hidden / 2 >= (1u << 31)))
-        tt = 4;
+    const bool fat_ok = hidden % 256 == 0 && (size_t)P * inter * 2 < (1u << 31) &&
+                        (size_t)n * hidden * 2 < (1u << 31) && (size_t)inter * hidden / 2 < (1u << 31);
+    if (tt == 8 && !fat_ok) tt = 4;
+    const bool split = fat_ok && grouped_splits(P, tt);
+    const long max_fat = split ? grouped_fat_tiles(P) : 0;
     const int trows = grouped_rows_per_tile(tt);
     size_t off = 0;
     auto take = [&](size_t b) { const size_t o = off; off += (b + 255) & ~(size_t)255; return o; };
     /* every bucket adds at most one partial tile, and every tile has a row */
     const long max_tiles = std::min(P, (P + trows - 1) / trows + n_experts);
-    const size_t o_grp = take((size_t)(n_experts + 1) * 4), o_tp = take((size_t)(n_experts + 1) * 4);
-    const size_t o_tg = take((size_t)(max_tiles + 4) * sizeof(TileRec));
+    const size_t o_grp = take((size_t)(n_experts + 1) * 4), o_tp = take((size_t)(n_experts + 2) * 4);
+    const size_t o_tg = take((size_t)(max_tiles + max_fat + 4) * sizeof(TileRec));
     const size_t o_pos = take((size_t)P * 4), o_row = take((size_t)P * 4);
     const size_t o_ch = take(route_chist_bytes(P, n_experts));
     const size_t o_x16 = take((size_t)n * hidden * 2), o_mid = take((size_t)P * inter * 2);
@@ -1611,6 +1613,9 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     ra.row_k = nullptr;
     ra.chist = (int *)(ws + o_ch);
     ra.status = g.st;
+    if (split) {
+        ra.fat_rows = GROUPED_FAT_ROWS; ra.fat_min = GROUPED_FAT_MIN; ra.fat_base = (int)max_tiles;
+    }
     /* The side stream starts where the call did (before the router, when that
      * is part of it) and needs nothing but x: it converts x to fp16, runs the
      * shared expert and is joined before the combine. A large x is converted
@@ -1649,10 +1654,21 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     ga.table = table; ga.n_experts = n_experts; ga.grp_off = grp; ga.tile_pre = tp; ga.tile_rec = tg;
     ga.row_tok = row; ga.nrows = n; ga.B = x16; ga.bexp = ex; ga.K = hidden; ga.N = inter;
     ga.out = mid; ga.limit = limit; ga.status = g.st;
-    HIPCHK(grouped_launch(FMT_FP4_E8M0, true, tt, ga, max_tiles, st), "routed gate/up launch");
+    /* a large bucket's tiles are the 128-row kernel's */
+    auto routed = [&](bool swiglu, const char *what) {
+        if (split) {
+            GroupedArgs fa = ga;
+            fa.tile_pre = tp + 1;
+            fa.tile_rec = tg + max_tiles;
+            HIPCHK(grouped_launch(FMT_FP4_E8M0, swiglu, 8, fa, max_fat, st), what);
+        }
+        HIPCHK(grouped_launch(FMT_FP4_E8M0, swiglu, tt, ga, max_tiles, st), what);
+        return 0;
+    };
+    if (routed(true, "routed gate/up launch")) return -1;
     ga.row_tok = nullptr; ga.bexp = nullptr;
     ga.nrows = (int)P; ga.B = mid; ga.K = inter; ga.N = hidden; ga.out = y;
-    HIPCHK(grouped_launch(FMT_FP4_E8M0, false, tt, ga, max_tiles, st), "routed down launch");
+    if (routed(false, "routed down launch")) return -1;
 
     if (shared) HIPCHK(hipStreamWaitEvent(st, g.join, 0), "join wait");
     CombineArgs ca;

@@ -19,6 +19,9 @@ int c_dense8_tile(int M, long slabs) { long c = 0; return dense8_tile(M, slabs, 
 int c_mmq_takes_seam(int nt, int rows, int dense) { return mmq_takes_seam(nt, rows, dense != 0); }
 int c_grouped_form(long pairs, int ne, int hidden, int inter, int stream)
 { return grouped_form(pairs, ne, hidden, inter, stream != 0); }
+int c_grouped_splits(long pairs, int form) { return grouped_splits(pairs, form); }
+long c_grouped_fat_tiles(long pairs) { return grouped_fat_tiles(pairs); }
+int c_fat(int which) { return which ? GROUPED_FAT_MIN : GROUPED_FAT_ROWS; }
 int c_bf16_form(int rows, int nt) { return bf16_form(rows, nt); }
 }
 """
@@ -35,6 +38,8 @@ def rules(tmp_path_factory):
                     os.path.join(PKG_DIR, "csrc"), str(src), "-o", str(so)], check=True)
     lib = C.CDLL(str(so))
     lib.c_dense8_tile.argtypes = [C.c_int, C.c_long]
+    lib.c_grouped_splits.argtypes = [C.c_long, C.c_int]
+    lib.c_grouped_fat_tiles.argtypes, lib.c_grouped_fat_tiles.restype = [C.c_long], C.c_long
     lib.c_grouped_form.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int]
     return lib
 
@@ -71,6 +76,26 @@ def test_expert_tiles_few_experts(rules, pairs, experts, hidden, inter, form):
     """A few experts' 128-row tiles leave the device idle: 16-row tiles until
     there are pairs enough."""
     assert rules.c_grouped_form(pairs, experts, hidden, inter, 1) == form
+
+
+def test_large_buckets_leave_the_16_row_tiles(rules):
+    """Above 4,096 pairs, whatever the mean bucket: 6,000 pairs may sit on 8 of
+    256 experts."""
+    for pairs, experts, inter in ((4206, 256, 2048), (6000, 256, 2048), (7168, 256, 2048), (8000, 512, 512)):
+        form = rules.c_grouped_form(pairs, experts, 4096, inter, 1)
+        assert form in (1, STREAM) and rules.c_grouped_splits(pairs, form)
+    assert not rules.c_grouped_splits(4096, STREAM)
+    assert not rules.c_grouped_splits(9000, 8)
+
+
+def test_fat_tile_bound(rules):
+    """The room for the large buckets' tile records holds their tiles, whatever
+    the buckets: each bucket's alone, and the one that fits least."""
+    rows, least = rules.c_fat(0), rules.c_fat(1)
+    worst = min(range(least + 1, 40 * rows), key=lambda c: c / -(-c // rows))
+    for c in range(least + 1, 40 * rows):
+        for m in (1, 7):                       # m buckets of c rows and one of the worst kind
+            assert m * -(-c // rows) + -(-worst // rows) <= rules.c_grouped_fat_tiles(m * c + worst)
 
 
 @pytest.mark.parametrize("rows,tokens,form", [

@@ -494,6 +494,35 @@ def test_grouped_stream_tiles(lib, pkg, oracle, counts, hidden, inter):
     assert e <= REL_L2_TOL, f"rel L2 {e:.3e} (max abs {max_abs(got, want):.3e})"
 
 
+@pytest.mark.parametrize("experts,hidden,inter", [(160, 1024, 1024), (300, 512, 256)])    # streaming, LDS-staged
+def test_grouped_large_buckets_split(lib, pkg, oracle, experts, hidden, inter):
+    """More than 4096 pairs at a small mean bucket: buckets of more than 64 rows
+    take 128-row tiles, the others 16-row ones (buckets around both limits and
+    around a tile's end, one of most pairs). Every token has the bits that it
+    has in a call of fewer pairs, where all tiles are of 16 rows; some against
+    the oracle."""
+    few = [DevExpert(lib, pkg, "fp4", inter, hidden, torch.Generator(device=DEV).manual_seed(e)) for e in range(5)]
+    counts = [64, 65, 0, 128, 129, 1, 256, 257, 16, 17, 63, 66, 320] + [5] * (experts - 14)
+    counts += [4300 - sum(counts)]
+    ids = np.concatenate([np.full(c, e, np.int32) for e, c in enumerate(counts)])
+    np.random.default_rng(experts).shuffle(ids)
+    n = len(ids)
+    assert n == 4300 and counts[-1] > 1000
+    x = bf16_rows(torch.Generator().manual_seed(hidden), n, hidden)
+    idx, w = ids.reshape(n, 1), np.ones((n, 1), np.float32)
+    table = [few[e % 5] for e in range(experts)]
+    lib.status()
+    got = run_dev(lib, table, None, x, idx, w, hidden, inter)
+    for lo in range(0, n, 2150):
+        part = slice(lo, lo + 2150)
+        assert np.array_equal(bits(got[part]), bits(run_dev(lib, table, None, x[part], idx[part], w[part], hidden, inter)))
+    assert lib.status() == 0
+    tokens = [int(np.flatnonzero(ids == e)[-1]) for e in range(len(counts)) if counts[e]][:20] + [n - 1]
+    want = oracle_tokens(oracle, table, None, x, idx, w, tokens)
+    e = rel_l2(got[tokens], want)
+    assert e <= REL_L2_TOL, f"rel L2 {e:.3e} (max abs {max_abs(got[tokens], want):.3e})"
+
+
 @pytest.mark.parametrize("mat,at", [(0, 5), (1, 1024 * 32 - 1), (2, 1024 * 16 + 3)])
 def test_grouped_stream_scale_range_flag(lib, pkg, mat, at):
     """A scale byte outside 104..140 in any matrix raises status bit 2, an
