@@ -137,6 +137,17 @@ inline bool grouped_splits(long pairs, int form) { return pairs > GROUPED_FEW_PA
 /* their number at most: such a bucket's tiles hold 64.5 rows each or more */
 inline long grouped_fat_tiles(long pairs) { return 2 * pairs / (GROUPED_FAT_ROWS + 1); }
 
+/* ---- routed MXFP8 experts (dsv4_moe_mx.hip) ---- */
+
+/* Whether rows of K columns take mx_tile_wide (else mx_tile, the same bits):
+ * whole groups of four stages, and enough of them for its longer start. us of
+ * the call, mx_tile / mx_tile_wide in both launches: 512 x 512, 16 experts,
+ * 2,000 tokens x 4 80.4 / 83.1; 1024 x 1024 118.8 / 119.0; 1536 x 1536 145.4 /
+ * 146.3; 32 experts, 4,000 tokens: 2048 x 2048 352 / 347, 3072 x 3072 637 / 603,
+ * 4096 x 2048 547 / 526. */
+constexpr int MX_WIDE_MIN_K = 2048;
+constexpr bool mx_wide_k(int K) { return K % 512 == 0 && K >= MX_WIDE_MIN_K; }
+
 /* ---- BF16 matvecs (dsv4_gemv.hip) ---- */
 
 /* LDS of k_gemv4_bf16: four rows and up to four tokens, 4,096 columns at a

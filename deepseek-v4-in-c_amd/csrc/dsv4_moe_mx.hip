@@ -49,7 +49,8 @@
  *   32,000 rows x 32 experts, hidden 4096, inter 2048: the call 1,046 -> 994
  *   us (scales 1,017 -> 992); 2,000 tokens x 128 experts 764 -> 694; 4,096
  *   tokens (Zipf) 1,404 -> 1,353. Rows whose scales start off a 16-byte
- *   boundary or are no multiple of four stages take mx_tile, a dword a row.
+ *   boundary, short ones and those of no multiple of four stages (mx_wide_k)
+ *   take mx_tile, a dword a row.
  *   Fewer L2 misses (units of 4 tiles x 8 slabs on an XCD: 10.4 -> 6.5 M)
  *   did not pay: the call +20 to +50 us.
  *
@@ -683,7 +684,7 @@ __global__ __launch_bounds__(512) void k_grouped_mx(GroupedMxArgs a, int thin_ro
         mx_fill_bad<SWIGLU, FEAT, 512>(a, it);
         return;
     }
-    if (a.K % 512 == 0 && (((uintptr_t)m1.s | (SWIGLU ? (uintptr_t)m3.s : 0) | (uintptr_t)a.BS) & 15) == 0) {
+    if (mx_wide_k(a.K) && (((uintptr_t)m1.s | (SWIGLU ? (uintptr_t)m3.s : 0) | (uintptr_t)a.BS) & 15) == 0) {
         if (it.ntok <= 128) mx_tile_wide<SWIGLU, 128>(a, m1, m3, it.r0, it.ntok, it.f0, lds);
         else mx_tile_wide<SWIGLU, 256>(a, m1, m3, it.r0, it.ntok, it.f0, lds);
         return;

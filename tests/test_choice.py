@@ -22,6 +22,7 @@ int c_grouped_form(long pairs, int ne, int hidden, int inter, int stream)
 int c_grouped_splits(long pairs, int form) { return grouped_splits(pairs, form); }
 long c_grouped_fat_tiles(long pairs) { return grouped_fat_tiles(pairs); }
 int c_fat(int which) { return which ? GROUPED_FAT_MIN : GROUPED_FAT_ROWS; }
+int c_mx_wide_k(int K) { return mx_wide_k(K); }
 int c_bf16_form(int rows, int nt) { return bf16_form(rows, nt); }
 }
 """
@@ -96,6 +97,12 @@ def test_fat_tile_bound(rules):
     for c in range(least + 1, 40 * rows):
         for m in (1, 7):                       # m buckets of c rows and one of the worst kind
             assert m * -(-c // rows) + -(-worst // rows) <= rules.c_grouped_fat_tiles(m * c + worst)
+
+
+@pytest.mark.parametrize("cols,wide", [(512, 0), (1024, 0), (1536, 0), (2048, 1), (2304, 0), (2560, 1), (4096, 1)])
+def test_mx_scales_four_stages_at_a_time(rules, cols, wide):
+    """Only rows long enough for the wide form's start, and of whole groups."""
+    assert rules.c_mx_wide_k(cols) == wide
 
 
 @pytest.mark.parametrize("rows,tokens,form", [

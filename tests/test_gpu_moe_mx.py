@@ -236,12 +236,13 @@ def test_mx_shapes(lib, pkg, oracle, n, topk, ne, zipf, hidden, inter, with_shar
              tokens, smid=smid)
 
 
-@pytest.mark.parametrize("hidden,inter", [(512, 512), (1024, 1536), (4096, 512), (2048, 1024)])
+@pytest.mark.parametrize("hidden,inter", [(512, 512), (1024, 1536), (4096, 512), (2048, 1024), (512, 2048), (2560, 2560)])
 def test_mx_scale_loads_same_bits(lib, pkg, hidden, inter):
-    """Scales in 16-byte pieces of four stages give the bits of scales a dword
-    at a time, which experts whose scales start 4 bytes past a 16-byte
-    boundary take: buckets around every tile height, one group of stages and
-    more."""
+    """Scales in 16-byte pieces of four stages (rows of 2048 columns and more)
+    give the bits of scales a dword at a time, which shorter rows and experts
+    whose scales start 4 bytes past a 16-byte boundary take: buckets around
+    every tile height, in the gate/up launch, the down launch and both, an
+    even and an odd number of groups of stages."""
     counts = [1, 17, 65, 96, 127, 128, 129, 255, 256, 257, 420]
     dgen = torch.Generator(device=DEV).manual_seed(hidden + inter)
     experts = [DevExpert(lib, pkg, "fp4", inter, hidden, dgen) for _ in counts]
