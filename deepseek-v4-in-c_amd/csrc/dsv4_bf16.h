@@ -156,7 +156,7 @@ struct Bf16Tile {
  * runs four of the chains, one MFMA a step: lane i + 4 b + 16 k supplies row
  * i, token i of chain 4 b + w for wave w. */
 /* Returns the dot product of row row0 + lane / 16 and token t0 + lane % 4 in
- * wave 0's lanes with (lane & 12) == 0. lds: b4_lds_bytes(min(ntok, 4)). Rows
+ * wave 0's lanes with (lane & 12) == 0. lds: b4_lds_bytes(min(ntok, 4), cols). Rows
  * past the end repeat the last, tokens past the end give no result. */
 __device__ __forceinline__ double bf16_dot4(uint8_t *lds, const uint16_t *W, int row0, int rows, const float *x,
                                             int x_ld, int ntok, int cols)
@@ -165,7 +165,8 @@ __device__ __forceinline__ double bf16_dot4(uint8_t *lds, const uint16_t *W, int
     const int lane = threadIdx.x & 63, wv = wave_in_group();
     const int cols16 = cols / 16 * 16;
     const int i = lane & 3, b = (lane >> 2) & 3, k = lane >> 4;
-    uint8_t *xl = lds + 4 * B4_W_LD;
+    const int w_ld = b4_w_ld(cols), x_ldb = b4_x_ld(cols);
+    uint8_t *xl = lds + 4 * w_ld;
     double acc = 0.0;
     for (int c0 = 0; c0 < cols16; c0 += B4_COLS) {
         const int nc = min(B4_COLS, cols16 - c0);    /* columns of this part */
@@ -174,7 +175,7 @@ __device__ __forceinline__ double bf16_dot4(uint8_t *lds, const uint16_t *W, int
         const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(W + (size_t)min(row0 + wv, rows - 1) * cols + c0), (short)0, 2 * nc, 0x00020000);
         for (int m = 0; m < (nc + 511) / 512; m++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (bf_lds_t *)(lds + wv * B4_W_LD + 1024 * m), 16,
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (bf_lds_t *)(lds + wv * w_ld + 1024 * m), 16,
                                                      1024 * m + 16 * lane, 0, 0, 0);
         /* the tokens' pieces dealt to the waves */
         const int xm = (nc + 255) / 256;
@@ -182,12 +183,12 @@ __device__ __forceinline__ double bf16_dot4(uint8_t *lds, const uint16_t *W, int
             const int t = m / xm, p = m - t * xm;
             const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
                 (void *)(x + (size_t)t * x_ld + c0), (short)0, 4 * nc, 0x00020000);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (bf_lds_t *)(xl + t * B4_X_LD + 1024 * p), 16,
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (bf_lds_t *)(xl + t * x_ldb + 1024 * p), 16,
                                                      1024 * p + 16 * lane, 0, 0, 0);
         }
         __syncthreads();                             /* everything has landed */
-        const uint16_t *wl = (const uint16_t *)(lds + i * B4_W_LD) + 16 * k + 4 * b + wv;
-        const float *xr = (const float *)(xl + (i < ntok ? i : 0) * B4_X_LD) + 16 * k + 4 * b + wv;
+        const uint16_t *wl = (const uint16_t *)(lds + i * w_ld) + 16 * k + 4 * b + wv;
+        const float *xr = (const float *)(xl + (i < ntok ? i : 0) * x_ldb) + 16 * k + 4 * b + wv;
         /* eight steps' reads issued before the eight before them multiply;
          * columns past nc were loaded as zeros up to whole 512s (rows) and
          * 256s (tokens), both at least the last step's end */
@@ -229,6 +230,77 @@ __device__ __forceinline__ double bf16_dot4(uint8_t *lds, const uint16_t *W, int
         for (int e = cols16; e < cols; e++) v = fma(bf16_of(wr[e]), (double)x[(size_t)i * x_ld + e], v);
     }
     return v;
+}
+
+/* One wave, four rows, a token at a time: lane 16 r + c runs chain c of row r
+ * as its FMAs, over rows and token in LDS. */
+constexpr int bfw_row_ld(int kch) { return 1024 * kch + 64; }            /* bank offset */
+constexpr int bfw_lds_bytes(int kch) { return 4 * bfw_row_ld(kch) + 2048 * kch; }
+
+/* rows row0 .. row0 + 3 (the last repeated) of `rows` into LDS, KCH KiB each;
+ * the caller waits */
+template <int KCH>
+__device__ __forceinline__ void bfw_rows_to_lds(uint8_t *lds, const uint16_t *W, int row0, int rows, int cols, int lane)
+{
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(W + (size_t)min(row0 + r, rows - 1) * cols), (short)0, 2 * cols, 0x00020000);
+#pragma unroll
+        for (int k = 0; k < KCH; k++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (bf_lds_t *)(lds + r * bfw_row_ld(KCH) + 1024 * k), 16,
+                                                     1024 * k + 16 * lane, 0, 0, 0);
+    }
+}
+
+/* the token into LDS behind the rows; the caller waits */
+template <int KCH>
+__device__ __forceinline__ void bfw_x_to_lds(uint8_t *lds, const float *x, int cols, int lane)
+{
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, 4 * cols, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < 2 * KCH; k++)
+        if (256 * k < cols)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (bf_lds_t *)(lds + 4 * bfw_row_ld(KCH) + 1024 * k), 16,
+                                                     1024 * k + 16 * lane, 0, 0, 0);
+}
+
+/* The dot product of row lane / 16 and the token, in that group's first lane.
+ * The next eight steps' reads are issued before the eight before them add. */
+template <int KCH>
+__device__ __forceinline__ double bfw_dot(const uint8_t *lds, int cols, int lane)
+{
+    const int steps = cols / 16;
+    const uint16_t *wr = (const uint16_t *)(lds + (lane >> 4) * bfw_row_ld(KCH));
+    const float *xr = (const float *)(lds + 4 * bfw_row_ld(KCH));
+    const uint16_t *wl = wr + (lane & 15);
+    const float *xl = xr + (lane & 15);
+    double acc = 0.0;
+    uint16_t w[8];
+    float xv[8];
+    int s = 0;
+    if (steps >= 8) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) { w[i] = wl[16 * i]; xv[i] = xl[16 * i]; }
+        for (; s + 8 <= steps; s += 8) {
+            uint16_t wn[8];
+            float xn[8];
+            const int sn = s + 16 <= steps ? s + 8 : s;     /* the last round re-reads its own */
+#pragma unroll
+            for (int i = 0; i < 8; i++) { wn[i] = wl[16 * (sn + i)]; xn[i] = xl[16 * (sn + i)]; }
+#pragma unroll
+            for (int i = 0; i < 8; i++) acc = fma(bf16_of(w[i]), (double)xv[i], acc);
+#pragma unroll
+            for (int i = 0; i < 8; i++) { w[i] = wn[i]; xv[i] = xn[i]; }
+        }
+    }
+    for (; s < steps; s++) acc = fma(bf16_of(wl[16 * s]), (double)xl[16 * s], acc);
+    acc = acc + __shfl_down(acc, 4, 16);       /* lanes 0..3, 8..11: chain c + chain c + 4 */
+    acc = acc + __shfl_down(acc, 8, 16);       /* lanes 0..3: bb[c]                        */
+    acc = acc + __shfl_down(acc, 1, 16);       /* lanes 0, 2: bb[0] + bb[1], bb[2] + bb[3] */
+    acc = acc + __shfl_down(acc, 2, 16);
+    for (int e = 16 * steps; e < cols; e++) acc = fma(bf16_of(wr[e]), (double)xr[e], acc);
+    return acc;
 }
 
 } // namespace dsv4

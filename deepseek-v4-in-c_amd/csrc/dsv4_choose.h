@@ -150,11 +150,13 @@ constexpr bool mx_wide_k(int K) { return K % 512 == 0 && K >= MX_WIDE_MIN_K; }
 
 /* ---- BF16 matvecs (dsv4_gemv.hip) ---- */
 
-/* LDS of k_gemv4_bf16: four rows and up to four tokens, 4,096 columns at a
- * time, a bank offset behind each. */
+/* LDS of k_gemv4_bf16: four rows and up to four tokens of b4_cols(cols) columns
+ * at a time (whole load instructions of the rows), a bank offset behind each. */
 constexpr int B4_COLS = 4096;
-constexpr int B4_W_LD = 2 * B4_COLS + 64, B4_X_LD = 4 * B4_COLS + 16;
-constexpr int b4_lds_bytes(int ntok) { return 4 * B4_W_LD + ntok * B4_X_LD; }
+constexpr int b4_cols(int cols) { return cols < B4_COLS ? (cols + 511) / 512 * 512 : B4_COLS; }
+constexpr int b4_w_ld(int cols) { return 2 * b4_cols(cols) + 64; }
+constexpr int b4_x_ld(int cols) { return 4 * b4_cols(cols) + 16; }
+constexpr int b4_lds_bytes(int ntok, int cols) { return 4 * b4_w_ld(cols) + ntok * b4_x_ld(cols); }
 
 /* Which form, all with the same bits. us at 4096 columns for (small /
  * rows / GEMM), measured: 1 token: 1024 rows 6.4 / 20 / 15, 8192 rows 18.8 /
@@ -162,15 +164,33 @@ constexpr int b4_lds_bytes(int ntok) { return 4 * B4_W_LD + ntok * B4_X_LD; }
  * rows 20 / 31 / 16, 8192 rows 37 / 31 / 26, 32768 rows 147 / 61 / 88; 32
  * tokens: 256 rows 10.1 / - / 15, 1024 rows 36 / - / 15. So: the rows form
  * for a few tokens of a large matrix, the small form while its workgroups
- * run in at most three rounds of what LDS lets the device hold at once, else
- * the GEMM. */
-enum Bf16Form { BF16_SMALL = 1, BF16_ROWS, BF16_GEMM };
-inline Bf16Form bf16_form(int rows, int nt)
+ * run in at most three rounds of what LDS lets the device hold at once (rows of
+ * 4096 columns), else the GEMM.
+ *
+ * One token of short rows, and two of a middling number of them, leave most of
+ * an MFMA's columns and a workgroup's latency unused: a wave of its own for
+ * four rows. us of (wave / small / rows): 1 token 8192 x 440 3.8 / 5.6 / 6.6,
+ * 16384 x 1024 6.9 / 10.5 / 8.5, 100000 x 232 13.4 / 33 / 16, 4096 x 2024 5.7 /
+ * 7.0 / 14, but 16384 x 2024 18.7 / 19.8 / 16.3 and 4096 x 4096 15.2 / 10.0 /
+ * 21; 2 tokens 12000 x 768 6.8 / 7.8 / 7.6, but 16384 x 768 9.7 / 9.5 / 7.8 and
+ * 4096 x 440 5.0 / 4.6. Rows of up to 128 columns: 3 tokens, 12000 rows 4.1 /
+ * 5.9 / 3.5. */
+enum Bf16Form { BF16_SMALL = 1, BF16_ROWS, BF16_GEMM, BF16_WAVE };
+constexpr int BF16_WAVE_COLS = 2048;
+inline Bf16Form bf16_form(int rows, int cols, int nt)
 {
-    if (nt <= 4 && rows >= (nt == 1 ? 9216 : 12288)) return BF16_ROWS;
-    const int lds = b4_lds_bytes(nt < 4 ? nt : 4);
+    if (nt == 1 && cols > 64 && cols <= 1024 && rows >= 2048) return BF16_WAVE;
+    if (nt == 1 && cols <= BF16_WAVE_COLS && rows >= 3072 && rows < 8192) return BF16_WAVE;
+    if (nt == 2 && cols > 128 && cols <= 1024 && rows >= 5120 && rows < 14336) return BF16_WAVE;
+    if (nt <= 4 && rows >= (nt == 1 ? 9216 : cols <= 128 ? 4096 : 12288)) return BF16_ROWS;
+    const int lds = b4_lds_bytes(nt < 4 ? nt : 4, B4_COLS);
     return ceil_div(rows, 4) * ceil_div(nt, 4) <= 3 * CUS * (160 * 1024 / lds) ? BF16_SMALL : BF16_GEMM;
 }
+/* Steps of 64 columns that the rows form has in flight: fewer where a row is
+ * hardly longer than eight and the waves many. 2 tokens, 4 / 8 steps, us: 100000
+ * rows of 256 columns 13.2 / 16.9, 960 39.0 / 48.0 (2024, one token: 93.5 /
+ * 91.4), 60000 of 256 10.4 / 9.8. */
+constexpr int bf16_rows_depth(int rows, int cols) { return cols < 1024 && rows >= 65536 ? 4 : 8; }
 
 } // namespace dsv4
 

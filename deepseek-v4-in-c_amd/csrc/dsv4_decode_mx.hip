@@ -2110,7 +2110,7 @@ constexpr size_t gateup_px8_lds() { return (size_t)8 * NP * TAB_CHUNK + TAB_ZERO
 template <int FMT, int NP>
 hipError_t gate_route_gateup_k(const GateRouteArgs &r, const GateUpMxArgs &a, hipStream_t st)
 {
-    const size_t lds = std::max<size_t>(gateup_px8_lds<NP>(), b4_lds_bytes(1));
+    const size_t lds = std::max<size_t>(gateup_px8_lds<NP>(), b4_lds_bytes(1, r.cols));
     const int nroute = (r.n_experts + 3) / 4;
     hipLaunchKernelGGL((k_gate_route_gateup<FMT, NP>), dim3((unsigned)(nroute + a.inter / 8)), dim3(512), lds, st, r,
                        a, nroute);

@@ -194,7 +194,7 @@ __device__ __forceinline__ float ld_dev(__amdgpu_buffer_rsrc_t r, int byte_off)
 
 /* The decode step's gate matvec and router in one launch: workgroup r of
  * nblk computes gate rows 4 r .. 4 r + 3; the last to finish routes the token.
- * Four waves; lds: b4_lds_bytes(1). */
+ * Four waves; lds: b4_lds_bytes(1, a.cols). */
 template <int NJ>
 __device__ __forceinline__ void gate_route_group(const GateRouteArgs &a, unsigned nblk, uint8_t *lds)
 {

@@ -151,6 +151,25 @@ __global__ __launch_bounds__(256) void k_gemv_bf16(GemvBf16Args a)
     }
 }
 
+/* One or two tokens of short rows: a wave per four rows. Bound by latency, and
+ * by HBM with very many rows ([100000 x 1024], one token: 31 us, 6.5 TB/s; in the
+ * form above 37). */
+template <int KCH>
+__global__ __launch_bounds__(64) void k_gemv_wave_bf16(GemvBf16Args a)
+{
+    __shared__ __align__(16) uint8_t lds[bfw_lds_bytes(KCH)];
+    const int lane = threadIdx.x, r0 = 4 * blockIdx.x, row = r0 + (lane >> 4);
+    bfw_rows_to_lds<KCH>(lds, a.W, r0, a.rows, a.cols, lane);
+    for (int t = 0; t < a.nt; t++) {
+        /* a single wave: its reads of the token before are done */
+        bfw_x_to_lds<KCH>(lds, a.x + (size_t)t * a.x_ld, a.cols, lane);
+        __builtin_amdgcn_s_waitcnt(0x0F70);          /* vmcnt(0): rows and token landed */
+        asm volatile("" ::: "memory");
+        const double v = bfw_dot<KCH>(lds, a.cols, lane);
+        if ((lane & 15) == 0 && row < a.rows) a.y[(size_t)t * a.y_ld + row] = (float)v;
+    }
+}
+
 /* Few tokens, few rows: four rows and four tokens per workgroup. Bound by
  * latency: the [256 x 4096] gate, 8 tokens, 42.3 -> 6.8 us. */
 __global__ __launch_bounds__(256) void k_gemv4_bf16(GemvBf16Args a)
@@ -256,23 +275,33 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemvBf16Args a)
 hipError_t gemv_bf16_launch(const GemvBf16Args &a, hipStream_t st)
 {
     if (a.rows <= 0 || a.cols <= 0 || a.cols % 8 || a.nt <= 0) return hipErrorInvalidValue;
-    const Bf16Form form = bf16_form(a.rows, a.nt);
+    static_assert(BF16_WAVE_COLS == 4 * 512, "the longest rows of k_gemv_wave_bf16<4>");
+    const Bf16Form form = bf16_form(a.rows, a.cols, a.nt);
     if (form == BF16_ROWS) {
         constexpr int RG = 2;
         const int waves = (a.rows + 8 * RG - 1) / (8 * RG);
-        hipLaunchKernelGGL((k_gemv_bf16<RG, 8>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, a);
+        const dim3 grid((unsigned)((waves + 3) / 4));
+        if (bf16_rows_depth(a.rows, a.cols) == 4) hipLaunchKernelGGL((k_gemv_bf16<RG, 4>), grid, dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((k_gemv_bf16<RG, 8>), grid, dim3(256), 0, st, a);
+        return hipGetLastError();
+    }
+    if (form == BF16_WAVE) {
+        const dim3 grid((unsigned)((a.rows + 3) / 4));
+        if (a.cols <= 512) hipLaunchKernelGGL(k_gemv_wave_bf16<1>, grid, dim3(64), 0, st, a);
+        else if (a.cols <= 1024) hipLaunchKernelGGL(k_gemv_wave_bf16<2>, grid, dim3(64), 0, st, a);
+        else hipLaunchKernelGGL(k_gemv_wave_bf16<4>, grid, dim3(64), 0, st, a);
         return hipGetLastError();
     }
     if (form == BF16_SMALL) {
         static bool attr_done = false;             /* not again inside a stream capture of a later call */
         if (!attr_done) {
             const hipError_t e = hipFuncSetAttribute((const void *)k_gemv4_bf16,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, b4_lds_bytes(4));
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, b4_lds_bytes(4, B4_COLS));
             if (e != hipSuccess) return e;
             attr_done = true;
         }
         hipLaunchKernelGGL(k_gemv4_bf16, dim3((unsigned)((a.rows + 3) / 4), (unsigned)((a.nt + 3) / 4)), dim3(256),
-                           b4_lds_bytes(a.nt < 4 ? a.nt : 4), st, a);
+                           b4_lds_bytes(a.nt < 4 ? a.nt : 4, a.cols), st, a);
         return hipGetLastError();
     }
     const long grid = (((long)a.nt + 15) / 16) * (((long)a.rows + 15) / 16);

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void k_route(GateRouteArgs a)
 template <int NJ>
 __global__ __launch_bounds__(256) void k_gate_route_bf16(GateRouteArgs a)
 {
-    __shared__ __align__(16) uint8_t lds[b4_lds_bytes(1)];
+    __shared__ __align__(16) uint8_t lds[b4_lds_bytes(1, B4_COLS)];
     gate_route_group<NJ>(a, gridDim.x, lds);
 }
 

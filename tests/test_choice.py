@@ -23,11 +23,11 @@ int c_grouped_splits(long pairs, int form) { return grouped_splits(pairs, form);
 long c_grouped_fat_tiles(long pairs) { return grouped_fat_tiles(pairs); }
 int c_fat(int which) { return which ? GROUPED_FAT_MIN : GROUPED_FAT_ROWS; }
 int c_mx_wide_k(int K) { return mx_wide_k(K); }
-int c_bf16_form(int rows, int nt) { return bf16_form(rows, nt); }
+int c_bf16_form(int rows, int cols, int nt) { return bf16_form(rows, cols, nt); }
 }
 """
 STREAM = 5
-SMALL, ROWS, GEMM = 1, 2, 3
+SMALL, ROWS, GEMM, WAVE = 1, 2, 3, 4
 
 
 @pytest.fixture(scope="module")
@@ -105,8 +105,12 @@ def test_mx_scales_four_stages_at_a_time(rules, cols, wide):
     assert rules.c_mx_wide_k(cols) == wide
 
 
-@pytest.mark.parametrize("rows,tokens,form", [
-    (256, 1, SMALL), (256, 8, SMALL), (129280, 1, ROWS), (16384, 4, ROWS), (4096, 4, GEMM), (256, 700, GEMM),
+@pytest.mark.parametrize("rows,cols,tokens,form", [
+    (256, 4096, 1, SMALL), (256, 4096, 8, SMALL), (129280, 4096, 1, ROWS), (16384, 4096, 4, ROWS), (4096, 4096, 4, GEMM),
+    (256, 4096, 700, GEMM),
+    (8553, 440, 1, WAVE), (103825, 232, 1, WAVE), (8137, 2024, 1, WAVE), (5492, 544, 2, WAVE), (2048, 136, 1, WAVE),
+    (16384, 2024, 1, ROWS), (8192, 2056, 1, SMALL), (1024, 440, 1, SMALL), (16384, 768, 2, ROWS), (4096, 440, 2, SMALL),
+    (12000, 64, 3, ROWS), (12000, 136, 3, GEMM),
 ])
-def test_bf16_form(rules, rows, tokens, form):
-    assert rules.c_bf16_form(rows, tokens) == form
+def test_bf16_form(rules, rows, cols, tokens, form):
+    assert rules.c_bf16_form(rows, cols, tokens) == form

@@ -120,7 +120,11 @@ def test_bf16_gemv_special_values(lib, pkg, oracle, rows, cols, nt):
     (12287, 136, 3), (12301, 1096, 4), (12288, 24, 2),    # and from 12288 for two to four
     (5, 4104, 4), (6, 8192, 5), (30, 8184, 8), (4, 16, 1),      # small form: one and two parts of columns
     (2048, 264, 4), (2052, 264, 4), (1021, 264, 8),       # small form's and GEMM's sides of the three rounds
-    (17, 4104, 529), (3100, 264, 9), (3073, 520, 17), (3085, 8, 32)])
+    (17, 4104, 529), (3100, 264, 9), (3073, 520, 17), (3085, 8, 32),
+    (2049, 72, 1), (2050, 512, 1), (2051, 520, 1), (4099, 1024, 1), (3075, 1032, 1), (3073, 2048, 1),   # a wave per four rows
+    (5121, 136, 2), (5122, 1016, 2), (3077, 16, 1),
+    (65537, 136, 2), (65541, 272, 3), (65536, 1016, 4), (65539, 8, 1), (14337, 520, 2),   # rows form, four steps in flight
+    (4097, 80, 3), (12290, 1024, 2), (33, 504, 3), (34, 1032, 2)])                # and eight; small form of short rows
 def test_bf16_forms(lib, pkg, oracle, rows, cols, nt):
     """Each form of the BF16 matvec at its edges: rows and tokens past the
     last tile, one to three 16-column groups past the last 64, trailing 8
