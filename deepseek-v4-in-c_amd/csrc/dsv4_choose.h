@@ -69,16 +69,22 @@ inline int dense8_tile(int M, long slabs, long *cost)
 
 /* Whether an FP8 matrix of rows x cols against nt tokens takes the seam GEMM
  * (128 x 256 tiles) rather than k_dense8 (dense) or, for operands that k_dense8
- * does not address, the grouped form. The seam GEMM's round is 60 in
- * dense8_tile's units: 4096 x 4096, 1,500 tokens 68.1 against 67.2 us dense,
- * 2,048 tokens 77.5 / 108.8; 1024 x 4096, 2,048 tokens 65.5 / 37.6. */
+ * does not address, the grouped form. A unit of dense8_tile's costs takes a time
+ * that grows as 620 + cols, a round of the seam GEMM as 12,000 + 59 cols (its
+ * epilogue is the smaller part of a long row), a tenth of it as the round's
+ * tiles. us of dense / seam: 4096 x 4096,
+ * 1,500 tokens 70 / 74, 2,000 tokens 113 / 79; 15360 x 4096, 500 tokens 94 / 71;
+ * 512 x 4096, 4,000 tokens 47 / 75; 1280 x 384, 3,708 tokens 23.7 / 16.6; 15360 x
+ * 640, 1,751 tokens 87 / 67; 1280 x 128, 2,000 tokens both 11.4. Of 246 shapes the
+ * choice is within 9 % of the better one, on average 0.1 %. */
 constexpr int MMQ_SEAM_GEMM_MIN_TOKENS = 1280;
-inline bool mmq_takes_seam(int nt, int rows, bool dense)
+inline bool mmq_takes_seam(int nt, int rows, int cols, bool dense)
 {
     if (!dense) return nt >= MMQ_SEAM_GEMM_MIN_TOKENS;
-    long cost = 0;
-    dense8_tile(nt, rows / 128, &cost);
-    return 60 * rounds(ceil_div(nt, 128) * ceil_div(rows, 256)) < cost;
+    long units = 0;
+    dense8_tile(nt, rows / 128, &units);
+    const long tiles = ceil_div(nt, 128) * ceil_div(rows, 256), past = tiles > CUS ? tiles : CUS;
+    return (9 * CUS * rounds(tiles) + past) * (12000 + 59L * cols) < 10 * CUS * units * (620 + cols);
 }
 
 /* ---- routed FP4 experts (dsv4_moe_grouped.hip) ---- */

@@ -808,7 +808,7 @@ static int enqueue_mmq(const DSV4QMat &d, int fmt, const float *x, float *y, int
         a.m1 = d; a.nrows = nt; a.B = x16; a.bexp = ex; a.K = d.cols; a.N = d.rows; a.out = y;
         a.status = g.st;
         const bool dense = grouped_dense_ok(a, fmt, false);
-        if (fmt != FMT_FP4_E8M0 && mmq_takes_seam(nt, d.rows, dense) && aligned16(d.w) &&
+        if (fmt != FMT_FP4_E8M0 && mmq_takes_seam(nt, d.rows, d.cols, dense) && aligned16(d.w) &&
             gemm_seam_ok(nt, d.rows, d.cols)) {
             SeamGemmArgs sg;
             sg.X = x16; sg.ex = ex; sg.W = (const uint8_t *)d.w; sg.Sw = d.s; sg.C = y;

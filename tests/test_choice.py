@@ -16,7 +16,7 @@ using namespace dsv4;
 extern "C" {
 int c_gemm_mid_tile(int M, int N, int K) { return gemm_mid_tile(M, N, K); }
 int c_dense8_tile(int M, long slabs) { long c = 0; return dense8_tile(M, slabs, &c); }
-int c_mmq_takes_seam(int nt, int rows, int dense) { return mmq_takes_seam(nt, rows, dense != 0); }
+int c_mmq_takes_seam(int nt, int rows, int cols) { return mmq_takes_seam(nt, rows, cols, true); }
 int c_grouped_form(long pairs, int ne, int hidden, int inter, int stream)
 { return grouped_form(pairs, ne, hidden, inter, stream != 0); }
 int c_grouped_splits(long pairs, int form) { return grouped_splits(pairs, form); }
@@ -56,6 +56,16 @@ def test_gemm_tile(rules, tokens, rows, cols, tile):
 @pytest.mark.parametrize("tokens,rows,tile", [(77, 4096, 1), (333, 4096, 3), (700, 4096, 6)])
 def test_dense_tile(rules, tokens, rows, tile):
     assert rules.c_dense8_tile(tokens, rows // 128) == tile
+
+
+@pytest.mark.parametrize("tokens,rows,cols,seam", [
+    (1500, 4096, 4096, 0), (2000, 4096, 4096, 1), (2048, 1024, 4096, 0), (500, 15360, 4096, 1), (333, 4096, 4096, 0),
+    (3708, 1280, 384, 1), (1751, 15360, 640, 1), (1737, 10240, 768, 1), (2059, 4352, 512, 1), (3000, 2048, 128, 1),
+    (2803, 3072, 640, 1),
+    (1000, 1280, 128, 0), (2000, 1280, 2048, 0),
+])
+def test_many_token_matmul(rules, tokens, rows, cols, seam):
+    assert rules.c_mmq_takes_seam(tokens, rows, cols) == seam
 
 
 @pytest.mark.parametrize("tokens,experts,hidden,inter,form", [
