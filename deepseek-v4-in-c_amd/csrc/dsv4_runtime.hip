@@ -1587,11 +1587,12 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     const size_t o_x16 = take((size_t)n * hidden * 2), o_mid = take((size_t)P * inter * 2);
     const size_t o_y = take((size_t)P * hidden * 4), o_ex = take((size_t)n * 4);
     const bool fork_x = (size_t)n * hidden > ((size_t)1 << 22);
+    const bool x_first = shared && !fork_x && !forked;         /* converted ahead of the fork, see below */
     size_t o_smid = 0, o_ys = 0, o_sx = o_x16, o_sex = o_ex;   /* the side stream's x */
     if (shared) {
         o_smid = take((size_t)n * sinter * 2);
         o_ys = take((size_t)n * hidden * 4);
-        if (!fork_x) {
+        if (!fork_x && !x_first) {
             o_sx = take((size_t)n * hidden * 2);
             o_sex = take((size_t)n * 4);
         }
@@ -1616,22 +1617,31 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     if (split) {
         ra.fat_rows = GROUPED_FAT_ROWS; ra.fat_min = GROUPED_FAT_MIN; ra.fat_base = (int)max_tiles;
     }
-    /* The side stream starts where the call did (before the router, when that
-     * is part of it) and needs nothing but x: it converts x to fp16, runs the
-     * shared expert and is joined before the combine. A large x is converted
-     * only there, beside the routing permutation, and this stream waits for
-     * it before the routed launches; a small one is converted once more by
-     * workgroups of the permutation's launch, which spares that wait (about
-     * 6 us between two kernels of this stream) and the launch. With the
-     * router's own change: 7 tokens behind the router 135 -> 124 us, 20 tokens
-     * without a shared expert 237 -> 225, 64 tokens, routing known, 297 -> 295. */
+    /* The side stream runs the shared expert and is joined before the combine;
+     * it needs nothing but x as fp16. A large x is converted only there, beside
+     * the routing permutation, and this stream waits for it before the routed
+     * launches. A small one, by who is ahead:
+     *   behind a router the side stream starts where the call did and converts
+     *   for itself, the permutation's launch once more for this one in
+     *   workgroups of its own, which spares a wait (about 6 us between two
+     *   kernels of this stream) and a launch (7 tokens 135 -> 124 us);
+     *   with the routing known the routed launches would be on the CUs before
+     *   the side stream has waited and converted, and the shared expert, often
+     *   the longer chain, behind them: it is converted here first, then the
+     *   side stream starts beside the permutation (FP8 shared expert, 4096 x
+     *   2048, top-3 of 64, 4 tokens 66 us against 78 as behind a router, 4096 x
+     *   512, top-7 of 64, 20 tokens 62 / 74, 1024 x 1024, top-5 of 128, 179
+     *   tokens 75 / 80; the other way, top-6 of 256, 6 tokens 105 / 98);
+     *   without a shared expert the permutation's launch converts alone (20
+     *   tokens 237 -> 225). */
+    if (x_first) HIPCHK(to_f16_rows_launch(x16, ex, x, n, hidden, st), "x fp16 launch");
     if (shared || fork_x) {
         if (!forked) HIPCHK(hipEventRecord(g.fork, st), "fork record");
         HIPCHK(hipStreamWaitEvent(g.side, g.fork, 0), "fork wait");
-        HIPCHK(to_f16_rows_launch(sx16, sex, x, n, hidden, g.side), "x fp16 launch");
+        if (!x_first) HIPCHK(to_f16_rows_launch(sx16, sex, x, n, hidden, g.side), "x fp16 launch");
     }
     if (fork_x) HIPCHK(hipEventRecord(g.xq, g.side), "convert record");
-    RowsF16Args xa = {x16, ex, x, fork_x ? 0 : n, hidden};
+    RowsF16Args xa = {x16, ex, x, fork_x || x_first ? 0 : n, hidden};
     HIPCHK(moe_route_launch(ra, xa, st), "route launch");
     if (fork_x) HIPCHK(hipStreamWaitEvent(st, g.xq, 0), "convert wait");
 
