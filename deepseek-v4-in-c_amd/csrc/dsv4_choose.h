@@ -100,10 +100,12 @@ constexpr int GROUPED_STREAM = 5, GROUPED_DENSE = 6;
  * 1,128 of the 128-row tiles; at 33 rows an expert 1,233 / 1,374 / 1,193).
  * With fewer than four steps of 256 to a row its setup costs more than it
  * saves (inter 512: 62 against 59 us at 60 tokens): there the LDS-staged
- * tiles, 16 rows up to 16 rows an expert, else 128 rows (weights reused
- * across a tile; 64 experts, hidden 4096, inter 512: 60 tokens 89 against 101
- * us, 300 tokens 146 / 134, 700 tokens 223 / 187). stream: the geometry is one
- * that the streaming tiles take.
+ * tiles, 16 rows up to 32 rows an expert (16 beyond GROUPED_FEW_PAIRS), else
+ * 128 rows, which use the weights again across a tile. us of 16 / 128 rows with
+ * weights that no cache holds, as between a model's layers, and an FP8 shared
+ * expert: hidden 4096, inter 512, 64 experts, 17 rows each 120 / 132, 24 rows
+ * 134 / 140, 36 rows 156 / 156, 60 rows 208 / 183; 2048 x 512, 128 experts, 17
+ * rows 114 / 121. stream: the geometry is one that the streaming tiles take.
  *
  * Few experts make few 128-row tiles, and a workgroup of those takes its time
  * however many CUs stay idle: up to 4,096 pairs, where they do not fill the
@@ -118,7 +120,8 @@ constexpr long GROUPED_FEW_PAIRS = 4096;
 inline int grouped_form(long pairs, int n_experts, int hidden, int inter, bool stream)
 {
     const int form16 = stream && hidden >= 1024 && inter >= 1024 ? GROUPED_STREAM : 1;
-    if (pairs <= (form16 == GROUPED_STREAM ? 28L : 16L) * n_experts) return form16;
+    const long mean = form16 == GROUPED_STREAM ? 28 : pairs <= GROUPED_FEW_PAIRS ? 32 : 16;
+    if (pairs <= mean * n_experts) return form16;
     const double buckets = (double)(pairs < n_experts ? pairs : n_experts), rows = (double)pairs / buckets;
     const double tiles16 = (double)pairs / 16 + buckets / 2;
     const double tiles128 = rows > 64 ? (double)pairs / 128 + buckets / 2 : buckets;

@@ -82,6 +82,8 @@ def test_expert_tiles_top6(rules, tokens, experts, hidden, inter, form):
     (100, 1, 2048, 512, 1), (800, 1, 2048, 512, 1), (400, 8, 2048, 512, 1), (800, 2, 512, 512, 1),
     (4097, 1, 512, 512, 8),                                # past GROUPED_FEW_PAIRS
     (3200, 64, 4096, 2048, 8), (2240, 32, 2048, 512, 8),   # tiles enough for every CU
+    (1100, 64, 4096, 512, 1), (2048, 64, 4096, 512, 1), (2100, 64, 4096, 512, 8), (4096, 128, 2048, 512, 1),   # short rows
+    (4800, 256, 2048, 512, 8), (4800, 512, 2048, 512, 1),
 ])
 def test_expert_tiles_few_experts(rules, pairs, experts, hidden, inter, form):
     """A few experts' 128-row tiles leave the device idle: 16-row tiles until
