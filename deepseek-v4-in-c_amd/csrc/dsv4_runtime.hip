@@ -1552,10 +1552,11 @@ int dsv4_hip_gemm_mxfp8q_dev(void *C, int out_bf16, const uint8_t *Aq, const uin
  * in the dense tiles (701 tokens, the call: 890 -> 846 us, 2,048: 1,546 ->
  * 1,454; up to 192 the 16- and 64-row tiles disturb the routed launches less:
  * 150 tokens 446 against 451 us). */
+constexpr int SHARED_DENSE_MIN_TOKENS = 193;
 static int enqueue_dense(int fmt, bool swiglu, const GroupedArgs &a, hipStream_t st, const char *what)
 {
     int tt = a.nrows <= 64 ? 1 : 4;          /* enough workgroups for a small batch */
-    if (a.nrows > 192 && grouped_dense_ok(a, fmt, swiglu)) tt = GROUPED_DENSE;
+    if (a.nrows >= SHARED_DENSE_MIN_TOKENS && grouped_dense_ok(a, fmt, swiglu)) tt = GROUPED_DENSE;
     const long rows = tt == GROUPED_DENSE ? a.nrows : grouped_rows_per_tile(tt);
     HIPCHK(grouped_launch(fmt, swiglu, tt, a, (a.nrows + rows - 1) / rows, st), what);
     return 0;
@@ -1587,7 +1588,8 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     const size_t o_x16 = take((size_t)n * hidden * 2), o_mid = take((size_t)P * inter * 2);
     const size_t o_y = take((size_t)P * hidden * 4), o_ex = take((size_t)n * 4);
     const bool fork_x = (size_t)n * hidden > ((size_t)1 << 22);
-    const bool x_first = shared && !fork_x && !forked;         /* converted ahead of the fork, see below */
+    /* x converted ahead of the fork, see below */
+    const bool x_first = shared && !forked && !fork_x && n < SHARED_DENSE_MIN_TOKENS;
     size_t o_smid = 0, o_ys = 0, o_sx = o_x16, o_sex = o_ex;   /* the side stream's x */
     if (shared) {
         o_smid = take((size_t)n * sinter * 2);
@@ -1626,12 +1628,14 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
      *   workgroups of its own, which spares a wait (about 6 us between two
      *   kernels of this stream) and a launch (7 tokens 135 -> 124 us);
      *   with the routing known the routed launches would be on the CUs before
-     *   the side stream has waited and converted, and the shared expert, often
-     *   the longer chain, behind them: it is converted here first, then the
-     *   side stream starts beside the permutation (FP8 shared expert, 4096 x
-     *   2048, top-3 of 64, 4 tokens 66 us against 78 as behind a router, 4096 x
-     *   512, top-7 of 64, 20 tokens 62 / 74, 1024 x 1024, top-5 of 128, 179
-     *   tokens 75 / 80; the other way, top-6 of 256, 6 tokens 105 / 98);
+     *   the side stream has waited and converted, and the shared expert, a long
+     *   chain in its 16- and 64-row tiles, behind them: up to 192 tokens it is
+     *   converted here first, then the side stream starts beside the
+     *   permutation (FP8 shared expert, 4096 x 2048, top-3 of 64, 4 tokens 66 us
+     *   against 78 as behind a router, 4096 x 512, top-7 of 64, 20 tokens 62 /
+     *   74, 1024 x 1024, top-5 of 128, 179 tokens 75 / 80; the other way, top-6
+     *   of 256, 6 tokens 105 / 98). Beyond, in the dense tiles, as behind a
+     *   router (4096 x 512, top-4 of 32, 481 tokens 117 against 130);
      *   without a shared expert the permutation's launch converts alone (20
      *   tokens 237 -> 225). */
     if (x_first) HIPCHK(to_f16_rows_launch(x16, ex, x, n, hidden, st), "x fp16 launch");
