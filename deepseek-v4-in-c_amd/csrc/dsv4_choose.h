@@ -135,14 +135,21 @@ inline int grouped_form(long pairs, int n_experts, int hidden, int inter, bool s
  * weights the 16-row tiles would read and decode once per 16 of them: above
  * GROUPED_FEW_PAIRS pairs the buckets of more than GROUPED_FAT_MIN rows go to
  * 128-row tiles in launches of their own, ahead of the others on the stream
- * (where there are none, two launches of empty workgroups: 701 tokens, even
- * routing, 765 -> 769 us). 256 experts of 4096 x 2048, top-6, us without / with:
- * 1,000 tokens on 8 of them 578 / 359, on 64 660 / 435, Zipf 974 / 883; 701
- * tokens, Zipf, 819 / 784. Fat from 96 rows: 64 experts used 586, Zipf 880; the
- * others on a second stream beside them: Zipf 863, even routing 962 against
- * 955. Below, 16-row tiles alone are no slower (680 tokens on 8 experts: 390). */
+ * (where there are none, two launches of empty workgroups, 3 to 6 us). 256
+ * experts of 4096 x 2048, top-6, us without / with: 1,000 tokens on 8 of them
+ * 578 / 359, on 64 660 / 435, Zipf 974 / 883, even routing 942 / 949; 701
+ * tokens, Zipf, 819 / 784; of 2048 x 1024, 1,000 tokens on 8 175 / 140, Zipf 285
+ * / 297. Smaller experts are read again from the caches and keep one form (1024
+ * x 1024: on 8 109 / 91, but Zipf 163 / 173, even 166 / 171). Fat from 96 rows:
+ * 4096 x 2048, 64 experts used 586, Zipf 880; the others on a second stream
+ * beside them: Zipf 863, even routing 962 against 955. Below GROUPED_FEW_PAIRS
+ * 16-row tiles alone are no slower (680 tokens on 8 experts: 390). */
 constexpr int GROUPED_FAT_ROWS = 128, GROUPED_FAT_MIN = 64;
-inline bool grouped_splits(long pairs, int form) { return pairs > GROUPED_FEW_PAIRS && form != 8; }
+constexpr long GROUPED_FAT_WEIGHTS = 1L << 21;
+inline bool grouped_splits(long pairs, int form, int hidden, int inter)
+{
+    return pairs > GROUPED_FEW_PAIRS && form != 8 && (long)hidden * inter >= GROUPED_FAT_WEIGHTS;
+}
 /* their number at most: such a bucket's tiles hold 64.5 rows each or more */
 inline long grouped_fat_tiles(long pairs) { return 2 * pairs / (GROUPED_FAT_ROWS + 1); }
 

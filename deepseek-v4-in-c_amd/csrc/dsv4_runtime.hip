@@ -1574,7 +1574,7 @@ static int enqueue_moe_grouped(float *out, const float *x, int n, const DSV4Expe
     const bool fat_ok = hidden % 256 == 0 && (size_t)P * inter * 2 < (1u << 31) &&
                         (size_t)n * hidden * 2 < (1u << 31) && (size_t)inter * hidden / 2 < (1u << 31);
     if (tt == 8 && !fat_ok) tt = 4;
-    const bool split = fat_ok && grouped_splits(P, tt);
+    const bool split = fat_ok && grouped_splits(P, tt, hidden, inter);
     const long max_fat = split ? grouped_fat_tiles(P) : 0;
     const int trows = grouped_rows_per_tile(tt);
     size_t off = 0;

@@ -19,7 +19,7 @@ int c_dense8_tile(int M, long slabs) { long c = 0; return dense8_tile(M, slabs, 
 int c_mmq_takes_seam(int nt, int rows, int cols) { return mmq_takes_seam(nt, rows, cols, true); }
 int c_grouped_form(long pairs, int ne, int hidden, int inter, int stream)
 { return grouped_form(pairs, ne, hidden, inter, stream != 0); }
-int c_grouped_splits(long pairs, int form) { return grouped_splits(pairs, form); }
+int c_grouped_splits(long pairs, int form, int hidden, int inter) { return grouped_splits(pairs, form, hidden, inter); }
 long c_grouped_fat_tiles(long pairs) { return grouped_fat_tiles(pairs); }
 int c_fat(int which) { return which ? GROUPED_FAT_MIN : GROUPED_FAT_ROWS; }
 int c_mx_wide_k(int K) { return mx_wide_k(K); }
@@ -39,7 +39,7 @@ def rules(tmp_path_factory):
                     os.path.join(PKG_DIR, "csrc"), str(src), "-o", str(so)], check=True)
     lib = C.CDLL(str(so))
     lib.c_dense8_tile.argtypes = [C.c_int, C.c_long]
-    lib.c_grouped_splits.argtypes = [C.c_long, C.c_int]
+    lib.c_grouped_splits.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int]
     lib.c_grouped_fat_tiles.argtypes, lib.c_grouped_fat_tiles.restype = [C.c_long], C.c_long
     lib.c_grouped_form.argtypes = [C.c_long, C.c_int, C.c_int, C.c_int, C.c_int]
     return lib
@@ -96,9 +96,10 @@ def test_large_buckets_leave_the_16_row_tiles(rules):
     256 experts."""
     for pairs, experts, inter in ((4206, 256, 2048), (6000, 256, 2048), (7168, 256, 2048), (8000, 512, 512)):
         form = rules.c_grouped_form(pairs, experts, 4096, inter, 1)
-        assert form in (1, STREAM) and rules.c_grouped_splits(pairs, form)
-    assert not rules.c_grouped_splits(4096, STREAM)
-    assert not rules.c_grouped_splits(9000, 8)
+        assert form in (1, STREAM) and rules.c_grouped_splits(pairs, form, 4096, inter)
+    assert not rules.c_grouped_splits(4096, STREAM, 4096, 2048)
+    assert not rules.c_grouped_splits(9000, 8, 4096, 2048)
+    assert not rules.c_grouped_splits(6000, STREAM, 1024, 1024)      # small experts: from the caches
 
 
 def test_fat_tile_bound(rules):

@@ -494,7 +494,7 @@ def test_grouped_stream_tiles(lib, pkg, oracle, counts, hidden, inter):
     assert e <= REL_L2_TOL, f"rel L2 {e:.3e} (max abs {max_abs(got, want):.3e})"
 
 
-@pytest.mark.parametrize("experts,hidden,inter", [(160, 1024, 1024), (300, 512, 256)])    # streaming, LDS-staged
+@pytest.mark.parametrize("experts,hidden,inter", [(160, 2048, 1024), (300, 4096, 512)])    # streaming, LDS-staged
 def test_grouped_large_buckets_split(lib, pkg, oracle, experts, hidden, inter):
     """More than 4096 pairs at a small mean bucket: buckets of more than 64 rows
     take 128-row tiles, the others 16-row ones (buckets around both limits and
