@@ -1451,6 +1451,8 @@ __global__ __launch_bounds__(512) void k_gate_route_gateup(GateRouteArgs r, Gate
 {
     extern __shared__ __align__(16) uint8_t lds[];
     if ((int)blockIdx.x < nroute) {
+        /* waves 4 to 7 end here: s_barrier waits for the workgroup's waves that
+         * have not ended, so the router's barriers are among its four */
         if (threadIdx.x < 256) gate_route_group<4>(r, (unsigned)nroute, lds);
         return;
     }

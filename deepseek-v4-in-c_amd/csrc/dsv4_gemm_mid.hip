@@ -86,6 +86,7 @@ template <int T> struct Mid {
     static constexpr int LDS = NST * STAGE;
     static constexpr int LW = 16 / NWAVE, LX = 2 * T / NWAVE, VM = LW + LX + 1;
     static_assert(LX * NWAVE == 2 * T && (NST - 1) * VM < 64 && LDS <= 160 * 1024, "ring");
+    static_assert(U >= 2, "a stage's two weight operands are read beside the first two token groups");
 };
 
 template <int N>
@@ -194,7 +195,6 @@ __global__ __launch_bounds__(64 * Mid<T>::NWAVE) void k_gemm_mid(MidArgs a)
             const int u = q >> 1, i = q & 1;
             if (i == 0) read_x(nxt, buf, u);
             else if (u < 2) read_w(nxt, buf, u);
-            if (U == 1 && i == 1) read_w(nxt, buf, 1);
             if constexpr (MODE == T_MX) {
                 acc[i][u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
                     cur.w[i], cur.x[u], acc[i][u], 0, 0, 0, (int)swv, 0, (int)((cur.ts[u] >> (8 * gq)) & 0xFFu));

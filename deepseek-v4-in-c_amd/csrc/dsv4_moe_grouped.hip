@@ -1521,9 +1521,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
  * dense form in tiles of 128 weight rows x 16 T tokens. Products, order and
  * so bits are k_grouped2's.
  *
- * Eight waves, 4 x 32 rows (gate/up: 16 w1 rows and the w3 rows of the same
- * features) by 2 x 8 T tokens (T = 4, 6) or four by 16 T (T = 1 .. 3). A stage is one 128-wide reduction block, rows
- * and tokens by buffer loads straight to LDS, NST stages in a ring. A wave
+ * Four waves along the rows, 32 each (gate/up: 16 w1 rows and the w3 rows of
+ * the same features), by one over all 16 T tokens (T = 1 .. 3) or two over 8 T
+ * each (T = 4, 6). A stage is one 128-wide reduction block, rows and tokens by
+ * buffer loads straight to LDS, NST stages in a ring. A wave
  * reads its operands of the next stage while it multiplies one, a read to
  * two MFMAs and a load between them, so that the barrier between stages waits
  * for no read. A row block's scales sit in one register, one block per lane.
@@ -1800,25 +1801,16 @@ static hipError_t grouped2_ns(const GroupedArgs &a, long items, hipStream_t st)
     return hipGetLastError();
 }
 
-/* FP8 16-row tiles: when the grid outnumbers the CUs, two stages (2 x 40
- * KiB) so two workgroups share a CU (4096 x 4096 FP8 drop-in matmul, 192
- * tokens in 384 workgroups: 36.1 -> 29.7 us); up to one workgroup per CU the
- * three-stage ring keeps more of a lone workgroup's loads in flight (128
- * tokens 23.7 against 24.3 us, the batched decode's shared expert). */
+/* FP8 16-row tiles (a shared expert of up to 64 tokens): when the grid
+ * outnumbers the CUs, two stages (2 x 40 KiB) so two workgroups share a CU
+ * (hidden 4096, inter 6144, 64 tokens, the call 94 -> 80 us, inter 8192 122 ->
+ * 105); up to one workgroup per CU the three-stage ring keeps more of a lone
+ * workgroup's loads in flight (7168 x 4608, 34 tokens 81.5 against 85.5 us). */
 template <int WF, bool SW, int TT>
 static hipError_t grouped2(const GroupedArgs &a, long items, hipStream_t st)
 {
     if constexpr (WF != FMT_FP4_E8M0 && TT == 1) {
-        static int cus = 0;
-        if (cus == 0) {
-            int dev = 0;
-            if (hipGetDevice(&dev) != hipSuccess ||
-                hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-                (void)hipGetLastError();
-                cus = 256;
-            }
-        }
-        if (items > cus) return grouped2_ns<WF, SW, TT, 2>(a, items, st);
+        if (items > CUS) return grouped2_ns<WF, SW, TT, 2>(a, items, st);
     }
     return grouped2_ns<WF, SW, TT, g2_stages<WF, TT>()>(a, items, st);
 }

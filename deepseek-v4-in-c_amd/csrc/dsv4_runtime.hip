@@ -820,9 +820,9 @@ static int enqueue_mmq(const DSV4QMat &d, int fmt, const float *x, float *y, int
             HIPCHK(grouped_launch(fmt, false, GROUPED_DENSE, a, 1, st), "dense MFMA launch");
             return 0;
         }
-        /* 16-token tiles give a small batch more workgroups, 64-token tiles
-         * reuse each weight chunk more (4096 x 4096: 32 to 128 tokens 23 us
-         * against 28-32 in 64-token tiles, 256 tokens 37 against 33) */
+        /* 16-token tiles give a batch more workgroups, 64-token tiles reuse each
+         * weight chunk more (FP4 4096 x 4096, 16 / 64: 32 tokens 20.8 / 24.3 us,
+         * 192 tokens 25.1 / 34.0, and still 32.7 / 35.7 at 333) */
         const int tt = nt <= 192 ? 1 : 4;
         const long tiles = (nt + grouped_rows_per_tile(tt) - 1) / grouped_rows_per_tile(tt);
         HIPCHK(grouped_launch(fmt, false, tt, a, tiles, st), "dense MFMA launch");

@@ -68,6 +68,23 @@ def test_many_token_matmul(rules, tokens, rows, cols, seam):
     assert rules.c_mmq_takes_seam(tokens, rows, cols) == seam
 
 
+@pytest.mark.parametrize("rows,cols,tokens", [(3200, 256, 1280), (2432, 512, 1337), (2560, 1280, 1700), (2048, 128, 4096),
+                                              (2176, 640, 2050), (4224, 384, 1337)])
+def test_shapes_of_the_seam_tests(rules, rows, cols, tokens):
+    """The seam GEMM's GPU tests run it, and dense tiles beside it."""
+    assert rules.c_mmq_takes_seam(tokens, rows, cols) and not rules.c_mmq_takes_seam(500, rows, cols)
+
+
+def test_dense_tile_heights_of_the_seam_tests(rules):
+    """Every height among the cases of the same-bits test."""
+    cases = {(2048, 128): (32, 33, 129, 257, 300, 513, 600, 1000, 1290), (2176, 640): (32, 47, 300, 500, 700, 1290),
+             (4224, 384): (40, 500, 700)}
+    heights = {rules.c_dense8_tile(n, r // 128) for (r, c), ns in cases.items() for n in ns if not rules.c_mmq_takes_seam(n, r, c)}
+    assert heights == {1, 2, 3, 4, 6}
+    assert not rules.c_mmq_takes_seam(1290, 2560, 1280)
+    assert [rules.c_dense8_tile(n, 32) for n in (150, 96)] == [2, 1]
+
+
 @pytest.mark.parametrize("tokens,experts,hidden,inter,form", [
     (7, 256, 4096, 2048, STREAM), (64, 256, 4096, 2048, STREAM), (701, 256, 4096, 2048, STREAM),
     (1500, 256, 4096, 2048, 8), (60, 64, 4096, 512, 1), (700, 64, 4096, 512, 8),

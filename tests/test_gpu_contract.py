@@ -354,14 +354,15 @@ def _fp8_resident(lib, pkg, oracle, fmt, rng, rows, cols):
     return m, lambda x, nt: oracle.fp8f_n(W, S, x, rows, cols, 128, 128, nt)
 
 
+# matrices and token counts that take the seam GEMM, by the dispatch rule (test_choice.py asks it)
 @pytest.mark.parametrize("rows,cols,nt", [
-    (256, 1024, 1280),    # ten full 128-token tiles
-    (384, 512, 1337),     # a partial token tile and a 128-row feature tail
-    (1024, 2048, 1296),
+    (3200, 256, 1280),    # two reduction blocks, ten full token tiles, a 128-row feature tail
+    (2432, 512, 1337),    # four blocks, a partial token tile and a feature tail
+    (2560, 1280, 1700),   # ten blocks, whole feature tiles
 ])
 @pytest.mark.parametrize("fmt", ["fp8", "fp8f"])
 def test_seam_gemm_shapes(lib, pkg, oracle, rows, cols, nt, fmt):
-    """1280 tokens and more on FP8 weights: the GEMM-shaped seam kernel
+    """Many tokens on FP8 weights: the GEMM-shaped seam kernel
     (128 x 256 tiles, fp16 tokens, weights decoded in registers) against the
     oracle, every token within 1e-3."""
     rng = np.random.default_rng(rows + cols + nt + len(fmt))
@@ -377,12 +378,12 @@ def test_seam_gemm_shapes(lib, pkg, oracle, rows, cols, nt, fmt):
 
 @pytest.mark.parametrize("fmt", ["fp8", "fp8f"])
 def test_seam_gemm_bits_equal_grouped_form(lib, pkg, oracle, fmt):
-    """The seam kernel (1280 tokens, where the drop-in switches to it) and
-    the grouped kernel's dense form (1279 tokens) run the same MFMA steps and
-    block promotions: every one of the first 1279 tokens' outputs is bit for
-    bit the same in both, including rows beyond fp16 (|x| 1e5) and below its
-    normal range (1e-9)."""
-    rows, cols, nt = 512, 2048, 1280
+    """The seam kernel (1700 tokens of 2560 x 1280) and the dense tiles, which
+    have the grouped kernel's order (1290 tokens of the same matrix), run the
+    same MFMA steps and block promotions: every one of the first 1290 tokens'
+    outputs is bit for bit the same in both, including rows beyond fp16 (|x|
+    1e5) and below its normal range (1e-9)."""
+    rows, cols, nt, few = 2560, 1280, 1700, 1290
     rng = np.random.default_rng(128 + len(fmt))
     m, _ = _fp8_resident(lib, pkg, oracle, fmt, rng, rows, cols)
     x = rng.standard_normal((nt, cols)).astype(np.float32)
@@ -391,21 +392,22 @@ def test_seam_gemm_bits_equal_grouped_form(lib, pkg, oracle, fmt):
     x[2] = 0.0
     x = np.ascontiguousarray(x.reshape(-1))
     big = lib.mmq_n(m.desc, x, nt).reshape(nt, rows)
-    small = lib.mmq_n(m.desc, x, nt - 1).reshape(nt - 1, rows)
-    assert np.array_equal(bits(big[:nt - 1]), bits(small))
+    small = lib.mmq_n(m.desc, np.ascontiguousarray(x[:few * cols]), few).reshape(few, rows)
+    assert np.array_equal(bits(big[:few]), bits(small))
     m.drop()
 
 
 @pytest.mark.parametrize("fmt", ["fp8", "fp8f"])
 @pytest.mark.parametrize("rows,cols,tokens", [
     (2048, 128, (32, 33, 129, 257, 300, 513, 600, 1000, 1290, 4096)),     # every tile height, then 128 x 256
-    (2176, 640, (32, 47, 300, 500, 700, 1290)),                            # rows no multiple of eight tiles
+    (2176, 640, (32, 47, 300, 500, 700, 1290, 2050)),                      # rows no multiple of eight tiles, then a feature tail
+    (4224, 384, (40, 500, 700, 1337)),                                     # three blocks, the tallest dense tiles, seam
     (1024, 8192, (33, 600)),                                               # the longest rows of the dense tiles
-    (128, 8448, (40, 300, 1290)),                                          # past them: grouped form, 128 x 256
+    (128, 8448, (40, 300, 1290)),                                          # past 8192 bytes: the generic matvec throughout
 ])
 def test_seam_tile_sizes_same_bits(lib, pkg, oracle, rows, cols, tokens, fmt):
     """The forms of the FP8 seam give a token the same bits: the dense tiles of
-    16 to 96 tokens, the grouped form and the 128 x 256 tiles."""
+    16 to 96 tokens and the 128 x 256 tiles."""
     rng = np.random.default_rng(rows + cols + len(fmt))
     m, want_of = _fp8_resident(lib, pkg, oracle, fmt, rng, rows, cols)
     x = rng.standard_normal((tokens[-1], cols)).astype(np.float32)
@@ -424,10 +426,10 @@ def test_seam_tile_sizes_same_bits(lib, pkg, oracle, rows, cols, tokens, fmt):
 
 @pytest.mark.parametrize("fmt", ["fp8", "fp8f"])
 def test_fp8_16_token_tiles_ring_depths(lib, pkg, oracle, fmt):
-    """FP8 weights, 32-192 tokens: 16-token tiles with a two-stage ring when
-    the grid outnumbers the CUs (150 tokens x 4096 rows: 320 workgroups),
-    a three-stage ring otherwise (the first 96 tokens alone: 192). Against
-    the oracle, and the shared tokens bit for bit the same in both."""
+    """FP8 weights, 32 to a few hundred tokens: the dense tiles of 32 tokens
+    (150 tokens x 4096 rows; a three-stage ring) and of 16 (the first 96 tokens
+    alone; four stages). Against the oracle, and the shared tokens bit for bit
+    the same in both."""
     rows, cols, nt, nt_small = 4096, 1024, 150, 96
     rng = np.random.default_rng(150 + len(fmt))
     m, want_of = _fp8_resident(lib, pkg, oracle, fmt, rng, rows, cols)
@@ -468,7 +470,7 @@ def test_scale_byte_outside_fp16_range_returns_minus1(lib, pkg, oracle):
     m2.drop()
 
 
-@pytest.mark.parametrize("fmt,nt", [("fp8f", 40), ("fp4", 40), ("fp8f", 1288)])
+@pytest.mark.parametrize("fmt,nt", [("fp8f", 40), ("fp4", 40), ("fp8f", 1288)])     # dense tiles, grouped, dense
 def test_seam_large_and_tiny_rows(lib, pkg, oracle, fmt, nt):
     """The nt >= 32 seam on rows an unscaled fp16 cast would break: |x| up to
     1e5 (beyond fp16), rows scaled by 1e-9 (below fp16's normal range), an

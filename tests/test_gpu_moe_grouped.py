@@ -583,11 +583,14 @@ def test_grouped_misaligned_expert_flags_status(lib, pkg, counts, hidden, name, 
 
 
 @pytest.mark.parametrize("fmt", ["fp8f32", "fp8e8m0"])
-@pytest.mark.parametrize("hidden,inter,tokens", [(256, 2048, (64, 150, 193, 333, 450, 700)), (512, 640, (40, 210))])
+@pytest.mark.parametrize("hidden,inter,tokens", [(256, 2048, (64, 150, 193, 333, 450, 700)), (512, 640, (40, 210)),
+                                                 (768, 4352, (17, 64, 200))])
 def test_shared_tile_sizes_same_bits(lib, pkg, oracle, hidden, inter, tokens, fmt):
-    """An FP8 shared expert gives a token the same bits from the 16- and 64-row
-    tiles as from the dense tiles of 16 to 96 tokens above 192 tokens (the
-    routed expert's weight is zero, so the output is the shared one's)."""
+    """An FP8 shared expert gives a token the same bits from the 16-row tiles
+    (in a ring of three stages, or of two where they outnumber the CUs: 64
+    tokens of 4352 rows) and the 64-row tiles as from the dense tiles of 16 to
+    96 tokens above 192 tokens (the routed expert's weight is zero, so the
+    output is the shared one's)."""
     dgen = torch.Generator(device=DEV).manual_seed(hidden + inter)
     experts = [DevExpert(lib, pkg, "fp4", inter, hidden, dgen)]
     shared = DevExpert(lib, pkg, fmt, inter, hidden, dgen)
